@@ -82,7 +82,10 @@ static TileKernelChoice select_tile_kernel(uint32_t head_dim, uint32_t coordinat
             return {tile_map_kernel<128, 2, 8, 64, 4, 1, true>, 512, (uint32_t)TileSmem<128, 64, 4>::kBytes};
         }
         if (head_dim == 256) {
-            if (coordinates <= 64) return {tile_map_kernel<256, 1, 4, 32, 4, 1, true>, 256, (uint32_t)TileSmem<256, 32, 4, 256>::kBytes};   // raw codes in LDS
+            // Raw codes in LDS: 64 KB per block, so a compute unit has room for two, and a batch of 23 speculative requests on
+            // 1000..20000 tokens (Hq24/Hkv4, 434 MB) needs them: one block (294 registers, one wave per SIMD) leaves every
+            // wait of its tile chain bare, 180 us; two (222 registers) 112 us.
+            if (coordinates <= 64) return {tile_map_kernel<256, 1, 4, 32, 4, 2, true>, 256, (uint32_t)TileSmem<256, 32, 4, 256>::kBytes};
             if (coordinates <= 128) return {tile_map_kernel<256, 1, 8, 32, 4, 1, true>, 512, (uint32_t)TileSmem<256, 32, 4>::kBytes};
             return {tile_map_kernel<256, 2, 8, 32, 4, 1, true>, 512, (uint32_t)TileSmem<256, 32, 4>::kBytes};
         }
