@@ -127,10 +127,17 @@ static ReduceKernel select_reduce_rows_kernel(uint32_t head_dim, bool ranged) {
     return nullptr;
 }
 
-// Launches the Reduce over `units` tokens (flat) or Q ranges (ranged) of `max_q_tokens` token slots each.
-static void launch_reduce_kernel(const khm_gqa_sdpa_config& config, const khm_gqa_sdpa_shape& shape, bool ranged, uint32_t units,
-                                 uint32_t max_q_tokens, ReduceKernel sliced, const ReduceParams& p, hipStream_t stream) {
-    const bool few = (uint64_t)shape.num_total_sdpa_map_task_templates <= (uint64_t)kFewPartialsPerRow * units;
+// Extent of a padded domain that a launch has to cover: with a fixed active count the padding gets no blocks (they would
+// only read their count and leave, but each of them takes a slot first: 944 of 1024 templates of a block-drafting batch
+// are padding).  A replay parameter is not known until the kernel runs, so its launch covers the whole domain.
+static uint32_t launch_extent(khm_replay_u32 active, uint32_t total) { return active.is_parameter ? total : active.value; }
+
+// Launches the Reduce over the active ones of `total_units` tokens (flat) or Q ranges (ranged) of `max_q_tokens` token slots each.
+// Which kernel runs depends on the shape alone, so that a fixed and a replayed call give the same bits.
+static void launch_reduce_kernel(const khm_gqa_sdpa_config& config, const khm_gqa_sdpa_shape& shape, bool ranged, khm_replay_u32 num_active,
+                                 uint32_t total_units, uint32_t max_q_tokens, ReduceKernel sliced, const ReduceParams& p, hipStream_t stream) {
+    const bool few = (uint64_t)shape.num_total_sdpa_map_task_templates <= (uint64_t)kFewPartialsPerRow * total_units;
+    const uint32_t units = launch_extent(num_active, total_units);
     if (few) {
         const uint64_t rows = (uint64_t)units * max_q_tokens * config.num_q_heads;
         const uint32_t rows_per_block = kReduceThreads / (config.head_dim / 4);
@@ -393,7 +400,8 @@ static int launch_sliced_kv_map(const khm_sliced_kv* compute, const khm_sliced_k
         p.final_output = fused->final_output;
         p.gates = fused->gates;
     }
-    const dim3 grid(shape.num_total_sdpa_map_task_templates, config.num_kv_heads * compute->num_q_head_ranges, 1);
+    const dim3 grid(launch_extent(num_active_kv_splits, shape.num_total_sdpa_map_task_templates), config.num_kv_heads * compute->num_q_head_ranges, 1);
+    if (grid.x == 0) return KHM_OK;
     KHM_LAUNCH(compute->map, grid, dim3(kMapWaves * 64), 0, static_cast<hipStream_t>(stream), p);
     return check_launch("sliced-KV map");
 }
@@ -545,7 +553,7 @@ static int launch_sliced_kv_reduce(const khm_sliced_kv* compute, const khm_slice
     p.head_dim = config.head_dim;
     p.max_q_tokens = 1;
     p.partial_is_f32 = config.partial_dtype == KHM_DTYPE_F32;
-    launch_reduce_kernel(config, shape, false, shape.num_total_tokens, 1, compute->reduce, p, static_cast<hipStream_t>(stream));
+    launch_reduce_kernel(config, shape, false, num_active_tokens, shape.num_total_tokens, 1, compute->reduce, p, static_cast<hipStream_t>(stream));
     return check_launch("sliced-KV reduce");
 }
 
@@ -685,7 +693,9 @@ static int launch_sliced_q_map(const khm_sliced_q* compute, const khm_buffer& q,
         p.final_output = fused->final_output;
         p.gates = fused->gates;
     }
-    const dim3 grid(shape.num_total_sdpa_map_task_templates, config.num_kv_heads * compute->num_q_head_ranges, 1);
+    const dim3 grid(launch_extent(num_active_kv_splits, shape.num_total_sdpa_map_task_templates), config.num_kv_heads * compute->num_q_head_ranges, 1);
+    if (grid.x == 0) return KHM_OK;
+    KHM_REQUIRE((uint64_t)grid.x * grid.y <= 0xffffffffull, "GQA SplitKV SlicedQ map grid exceeds the u32 block domain");
     KHM_LAUNCH(compute->map, grid, dim3(compute->map_threads), compute->map_smem_bytes, static_cast<hipStream_t>(stream), p);
     return check_launch("sliced-Q map");
 }
@@ -805,7 +815,7 @@ static int sliced_q_reduce(const khm_sliced_q* compute, const khm_sliced_q_reduc
     p.partial_is_f32 = config.partial_dtype == KHM_DTYPE_F32;
     KHM_REQUIRE(!mul_overflows_u32(shape.num_total_q_token_tiles, compute->variant.map_max_q_tokens),
                 "GQA SplitKV SlicedQ reduce grid exceeds the u32 domain");
-    launch_reduce_kernel(config, shape, true, shape.num_total_q_token_tiles, compute->variant.map_max_q_tokens, compute->reduce, p,
+    launch_reduce_kernel(config, shape, true, num_active_q_token_tiles, shape.num_total_q_token_tiles, compute->variant.map_max_q_tokens, compute->reduce, p,
                          static_cast<hipStream_t>(stream));
     return check_launch("sliced-Q reduce");
 }

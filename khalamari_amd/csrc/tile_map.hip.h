@@ -16,7 +16,7 @@
 // passing through registers; NSTAGES tiles are in flight and one barrier per tile publishes them.  A direct load
 // writes 64 consecutive 16-byte chunks, so rows cannot be padded; instead each lane fetches the chunk whose index is
 // XOR-swizzled with the row, which makes both the b128 K reads and the transposed V reads bank-conflict free.
-// Blocks are renumbered so that each XCD walks a contiguous run of the (KV head, template) list: the Q ranges of
+// Blocks are renumbered so that each XCD walks a contiguous run of the (KV head, active template) list: the Q ranges of
 // one sequence share their K/V through that XCD's L2 instead of each pulling it from HBM.
 #pragma once
 #include <hip/hip_runtime.h>
@@ -185,33 +185,17 @@ void tile_map_kernel(const MapParams p) {
     const int r16 = lane & 15;
     const int g = lane >> 4;
 
-    // ---- XCD-aware block renumbering -------------------------------------------------------------------
-    // Hardware deals consecutive block ids round-robin to the 8 XCDs.  Work item w = (head group, template)
-    // in head-group-major order; XCD x takes the contiguous run [x * N / 8, (x + 1) * N / 8).
-    const uint32_t num_tasks = gridDim.x;
-    const uint32_t num_head_groups = gridDim.y;
-    const uint64_t total = (uint64_t)num_tasks * num_head_groups;
-    const uint64_t linear = (uint64_t)blockIdx.y * num_tasks + blockIdx.x;
-    uint64_t work = linear;
-    {
-        const uint64_t per_xcd = total / 8;
-        const uint64_t main = per_xcd * 8;
-        if (linear < main) work = (linear % 8) * per_xcd + linear / 8;
-    }
-    const uint32_t head_group = (uint32_t)(work / num_tasks);
-    // Templates are taken last to first: within a request the later Q ranges see more keys, so the long blocks start
-    // early and the short ones fill the end of the launch (2 % on a batch of 2048-token chunks).
-    const uint32_t task = num_tasks - 1 - (uint32_t)(work % num_tasks);
-
     // ---- task decode (uniform) ---------------------------------------------------------------------------
-    // every link of the chain arguments -> template -> Q range -> request slot is a scalar load, and what hangs on the
-    // same link is requested together (see split_kv_map_kernel)
+    // every link of the chain arguments -> active counts -> template -> Q range -> request slot is a scalar load, and what
+    // hangs on the same link is requested together (see split_kv_map_kernel)
     fetch_all_arguments(p);
     const ReplayValues replay = resolve_replay_values(p);
+    const WorkItem item = sliced_q_work_item(replay.num_active_kv_splits);
+    if (!item.live) return;
+    const uint32_t head_group = item.head_group, task = item.task;
     const uint32_t range_index = load_uniform_u32(p.templates, 3 * (uint64_t)task);
     const uint32_t kv_begin = load_uniform_u32(p.templates, 3 * (uint64_t)task + 1);
     const uint32_t kv_end = load_uniform_u32(p.templates, 3 * (uint64_t)task + 2);
-    if (task >= replay.num_active_kv_splits) return;
     if (range_index >= replay.num_active_q_token_tiles) return;
     const uint32_t flat_begin = load_uniform_u32(p.q_token_ranges, 2 * (uint64_t)range_index);
     const uint32_t flat_end = load_uniform_u32(p.q_token_ranges, 2 * (uint64_t)range_index + 1);
