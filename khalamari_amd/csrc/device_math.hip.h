@@ -61,6 +61,13 @@ __device__ __forceinline__ ReplayValues resolve_replay_values(const MapParams& p
                         p.num_active_kv_splits.is_parameter ? d : p.num_active_kv_splits.value};
 }
 
+// The active template count by itself: a fixed one is an argument, and nothing waits for memory.
+__device__ __forceinline__ uint32_t active_kv_splits(const MapParams& p) {
+    uint32_t active = p.num_active_kv_splits.value;
+    if (p.num_active_kv_splits.is_parameter) active = load_uniform_u32(p.replay_parameters, active);
+    return active;
+}
+
 // Block -> (head group, template) of a sliced-Q launch over `active` templates: head groups fastest, templates last to first.
 // Hardware deals consecutive block ids round-robin to the 8 XCDs, so with 8 KV heads every XCD keeps one head and with 4 or
 // 2 two or four XCDs take turns with a head's templates: the Q ranges of one sequence share their K/V through an XCD's L2, and

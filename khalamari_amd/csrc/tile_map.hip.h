@@ -186,12 +186,12 @@ void tile_map_kernel(const MapParams p) {
     const int g = lane >> 4;
 
     // ---- task decode (uniform) ---------------------------------------------------------------------------
-    // every link of the chain arguments -> active counts -> template -> Q range -> request slot is a scalar load, and what
+    // every link of the chain arguments (-> replayed count) -> template -> Q range -> request slot is a scalar load, and what
     // hangs on the same link is requested together (see split_kv_map_kernel)
     fetch_all_arguments(p);
-    const ReplayValues replay = resolve_replay_values(p);
-    const WorkItem item = sliced_q_work_item(replay.num_active_kv_splits);
+    const WorkItem item = sliced_q_work_item(active_kv_splits(p));
     if (!item.live) return;
+    const ReplayValues replay = resolve_replay_values(p);
     const uint32_t head_group = item.head_group, task = item.task;
     const uint32_t range_index = load_uniform_u32(p.templates, 3 * (uint64_t)task);
     const uint32_t kv_begin = load_uniform_u32(p.templates, 3 * (uint64_t)task + 1);
