@@ -81,6 +81,7 @@ struct WorkItem {
     bool live;
 };
 __device__ __forceinline__ WorkItem sliced_q_work_item(uint32_t active) {
+    if (active > gridDim.x) active = gridDim.x;   // a replayed count beyond the shape reads no template behind the table
     const uint32_t linear = blockIdx.y * gridDim.x + blockIdx.x;
     const uint32_t rank = linear / gridDim.y;
     return WorkItem{linear - rank * gridDim.y, active - 1 - rank, rank < active};

@@ -70,3 +70,7 @@ def test_fixed_and_replayed_counts_give_the_same_bytes(device, hq, hkv, d, fp8, 
         assert torch.equal(fixed, replayed)
         helpers.assert_parity(gpu_runner.bf16_tensor_to_f32(fixed)[:tokens], expected[:tokens], f"{active_requests} requests")
         assert np.all(fixed[tokens:].cpu().numpy() == POISON)
+        if active_requests == 5 and not direct:
+            # a replayed count beyond the shape stands for the whole table: no template is read behind it, padding has no Q range
+            beyond = torch.tensor([tokens, tiles, total + 7, 0], dtype=torch.int32, device=device)
+            assert torch.equal(fixed, run(*(ReplayU32.parameter(i) for i in range(3)), beyond))
