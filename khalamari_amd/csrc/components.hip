@@ -118,13 +118,17 @@ static ReduceKernel select_reduce_kernel(uint32_t head_dim, bool ranged) {
     return nullptr;
 }
 
-// Rows with few partials merge faster one row per thread group (no LDS pass); the shape's average decides.
+// Rows with few partials merge faster one row per thread group (no LDS pass); the shape's average decides, and so it does
+// for the number of partials a row requests at once (four take 50 registers and leave eight waves per SIMD, sixteen 122 and
+// four waves).
 constexpr uint32_t kFewPartialsPerRow = 16;
+constexpr uint32_t kVeryFewPartialsPerRow = 4;
 
-static ReduceKernel select_reduce_rows_kernel(uint32_t head_dim, bool ranged) {
-    if (head_dim == 128) return ranged ? split_kv_reduce_rows_kernel<128, true> : split_kv_reduce_rows_kernel<128, false>;
-    if (head_dim == 256) return ranged ? split_kv_reduce_rows_kernel<256, true> : split_kv_reduce_rows_kernel<256, false>;
-    return nullptr;
+typedef void (*ReduceRowsKernel)(const ReduceParams, uint32_t);
+template <int D>
+static ReduceRowsKernel reduce_rows_kernel_of(bool ranged, bool very_few) {
+    if (very_few) return ranged ? split_kv_reduce_rows_kernel<D, true, 4> : split_kv_reduce_rows_kernel<D, false, 4>;
+    return ranged ? split_kv_reduce_rows_kernel<D, true, 16> : split_kv_reduce_rows_kernel<D, false, 16>;
 }
 
 // Extent of a padded domain that a launch has to cover: with a fixed active count the padding gets no blocks (they would
@@ -136,13 +140,14 @@ static uint32_t launch_extent(khm_replay_u32 active, uint32_t total) { return ac
 // Which kernel runs depends on the shape alone, so that a fixed and a replayed call give the same bits.
 static void launch_reduce_kernel(const khm_gqa_sdpa_config& config, const khm_gqa_sdpa_shape& shape, bool ranged, khm_replay_u32 num_active,
                                  uint32_t total_units, uint32_t max_q_tokens, ReduceKernel sliced, const ReduceParams& p, hipStream_t stream) {
-    const bool few = (uint64_t)shape.num_total_sdpa_map_task_templates <= (uint64_t)kFewPartialsPerRow * total_units;
+    auto average_at_most = [&](uint32_t partials) { return (uint64_t)shape.num_total_sdpa_map_task_templates <= (uint64_t)partials * total_units; };
     const uint32_t units = launch_extent(num_active, total_units);
-    if (few) {
-        const uint64_t rows = (uint64_t)units * max_q_tokens * config.num_q_heads;
-        const uint32_t rows_per_block = kReduceThreads / (config.head_dim / 4);
-        KHM_LAUNCH(select_reduce_rows_kernel(config.head_dim, ranged), dim3((uint32_t)((rows + rows_per_block - 1) / rows_per_block)),
-                           dim3(kReduceThreads), 0, stream, p);
+    if (average_at_most(kFewPartialsPerRow)) {
+        const bool very_few = average_at_most(kVeryFewPartialsPerRow);
+        const uint32_t rows_per_block = kReduceThreads / (config.head_dim / 8);
+        const uint32_t blocks_per_unit = (uint32_t)(((uint64_t)max_q_tokens * config.num_q_heads + rows_per_block - 1) / rows_per_block);
+        const ReduceRowsKernel rows = config.head_dim == 128 ? reduce_rows_kernel_of<128>(ranged, very_few) : reduce_rows_kernel_of<256>(ranged, very_few);
+        KHM_LAUNCH(rows, dim3(units * blocks_per_unit), dim3(kReduceThreads), 0, stream, p, blocks_per_unit);
     } else {
         KHM_LAUNCH(sliced, dim3(units * max_q_tokens, config.num_q_heads, 1), dim3(kReduceThreads), 0, stream, p);
     }

@@ -12,13 +12,41 @@
 
 namespace khm {
 
-struct MergeState {
+// QUADS groups of four consecutive dims per lane.
+template <int QUADS>
+struct MergeStateOf {
     float run_max;
     float run_sum;
-    f32x4 acc;
+    f32x4 acc[QUADS];
 };
+typedef MergeStateOf<1> MergeState;
 
-__device__ __forceinline__ MergeState merge_state_empty() { return MergeState{-INFINITY, 0.0f, f32x4{0.0f, 0.0f, 0.0f, 0.0f}}; }
+template <int QUADS = 1>
+__device__ __forceinline__ MergeStateOf<QUADS> merge_state_empty() {
+    MergeStateOf<QUADS> state;
+    state.run_max = -INFINITY;
+    state.run_sum = 0.0f;
+#pragma unroll
+    for (int i = 0; i < QUADS; ++i) state.acc[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    return state;
+}
+
+// One more partial: its maximum, its exp-sum (both checked here: an empty partial changes nothing) and its normalized values.
+template <int QUADS>
+__device__ __forceinline__ void merge_one_partial(MergeStateOf<QUADS>& state, float part_max, float part_sum, const f32x4 (&value)[QUADS]) {
+    if (!(part_sum > 0.0f) || !(fabsf(part_max) < INFINITY)) return;  // empty partial
+    const float next_max = fmaxf(state.run_max, part_max);
+    const float keep = fast_exp(state.run_max - next_max);  // 0 while run_max is still -inf
+    const float weight = fast_exp(part_max - next_max) * part_sum;
+    state.run_sum = state.run_sum * keep + weight;
+#pragma unroll
+    for (int i = 0; i < QUADS; ++i) state.acc[i] = state.acc[i] * keep + value[i] * weight;
+    state.run_max = next_max;
+}
+
+__device__ __forceinline__ f32x4 bf16x4_to_f32x4(uint32_t a, uint32_t b) {
+    return f32x4{bf16_bits_to_f32(a & 0xffffu), bf16_bits_to_f32(a >> 16), bf16_bits_to_f32(b & 0xffffu), bf16_bits_to_f32(b >> 16)};
+}
 
 template <bool COHERENT>
 __device__ __forceinline__ float merge_load_f32(const float* address) {
@@ -60,21 +88,47 @@ __device__ __forceinline__ void merge_partial_slice(MergeState& state, const flo
         }
 #pragma unroll
         for (int k = 0; k < BATCH; ++k) {
-            if (!(part_sum[k] > 0.0f) || !(fabsf(part_max[k]) < INFINITY)) continue;  // empty partial
-            f32x4 value;
+            f32x4 value[1];
             if (f32_partials) {
-                value = f32x4{__uint_as_float((uint32_t)lo[k]), __uint_as_float((uint32_t)(lo[k] >> 32)),
-                              __uint_as_float((uint32_t)hi[k]), __uint_as_float((uint32_t)(hi[k] >> 32))};
+                value[0] = f32x4{__uint_as_float((uint32_t)lo[k]), __uint_as_float((uint32_t)(lo[k] >> 32)),
+                                 __uint_as_float((uint32_t)hi[k]), __uint_as_float((uint32_t)(hi[k] >> 32))};
             } else {
-                const uint32_t a = (uint32_t)lo[k], b = (uint32_t)(lo[k] >> 32);
-                value = f32x4{bf16_bits_to_f32(a & 0xffffu), bf16_bits_to_f32(a >> 16), bf16_bits_to_f32(b & 0xffffu), bf16_bits_to_f32(b >> 16)};
+                value[0] = bf16x4_to_f32x4((uint32_t)lo[k], (uint32_t)(lo[k] >> 32));
             }
-            const float next_max = fmaxf(state.run_max, part_max[k]);
-            const float keep = fast_exp(state.run_max - next_max);  // 0 while run_max is still -inf
-            const float weight = fast_exp(part_max[k] - next_max) * part_sum[k];
-            state.run_sum = state.run_sum * keep + weight;
-            state.acc = state.acc * keep + value * weight;
-            state.run_max = next_max;
+            merge_one_partial(state, part_max[k], part_sum[k], value);
+        }
+    }
+}
+
+// Merges the partials [begin, end) of one row, eight dims per lane (dims octet * 8 .. + 8), BATCH partials requested at once.
+// `row0` is the row of partial 0, `row_step` the rows from one partial to the next.
+template <int D, bool F32, int BATCH>
+__device__ __forceinline__ void merge_partial_octets(MergeStateOf<2>& state, const float* max_logits, const float* exp_sums, const void* partial,
+                                                     uint32_t begin, uint32_t end, uint64_t row0, uint64_t row_step, int octet) {
+    for (uint32_t first = begin; first < end; first += BATCH) {
+        float part_max[BATCH], part_sum[BATCH];
+        uint4 bits[BATCH], more[F32 ? BATCH : 1];
+#pragma unroll
+        for (int k = 0; k < BATCH; ++k) {
+            const bool ok = first + k < end;
+            const uint64_t row = row0 + (ok ? first + k : begin) * row_step;
+            part_max[k] = max_logits[row];
+            part_sum[k] = ok ? exp_sums[row] : 0.0f;
+            const uint4* source = reinterpret_cast<const uint4*>(reinterpret_cast<const unsigned char*>(partial) + (row * D + octet * 8) * (F32 ? 4 : 2));
+            bits[k] = source[0];
+            if constexpr (F32) more[k] = source[1];
+        }
+#pragma unroll
+        for (int k = 0; k < BATCH; ++k) {
+            f32x4 value[2];
+            if constexpr (F32) {
+                value[0] = __builtin_bit_cast(f32x4, bits[k]);
+                value[1] = __builtin_bit_cast(f32x4, more[k]);
+            } else {
+                value[0] = bf16x4_to_f32x4(bits[k].x, bits[k].y);
+                value[1] = bf16x4_to_f32x4(bits[k].z, bits[k].w);
+            }
+            merge_one_partial(state, part_max[k], part_sum[k], value);
         }
     }
 }
@@ -91,19 +145,30 @@ __device__ __forceinline__ MergeState merge_combine_slices(const float* stats, c
         if (slice_sum > 0.0f) {
             const float factor = fast_exp(stats[(first + i) * 2] - all_max);
             out.run_sum += slice_sum * factor;
-            out.acc += *reinterpret_cast<const f32x4*>(acc + (first + i) * D + chunk * 4) * factor;
+            out.acc[0] += *reinterpret_cast<const f32x4*>(acc + (first + i) * D + chunk * 4) * factor;
         }
     }
     return out;
 }
 
-// Normalizes, applies the optional bf16 gate (gqa_activation_gate.metal:19-39) and stores four bf16 outputs.
-__device__ __forceinline__ void merge_store_output(const MergeState& state, uint16_t* output, const uint16_t* gates, uint64_t out_index) {
-    f32x4 result = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (state.run_sum > 0.0f) result = state.acc / state.run_sum;
-    if (gates != nullptr) result = gate_bf16x4(result, gates + out_index);
-    const uint2 packed = make_uint2(pack_bf16x2(result[0], result[1]), pack_bf16x2(result[2], result[3]));
-    *reinterpret_cast<uint2*>(output + out_index) = packed;
+// Normalizes, applies the optional bf16 gate (gqa_activation_gate.metal:19-39) and stores four bf16 outputs per quad.
+template <int QUADS>
+__device__ __forceinline__ void merge_store_output(const MergeStateOf<QUADS>& state, uint16_t* output, const uint16_t* gates, uint64_t out_index) {
+    uint32_t words[2 * QUADS];
+#pragma unroll
+    for (int i = 0; i < QUADS; ++i) {
+        f32x4 result = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (state.run_sum > 0.0f) result = state.acc[i] / state.run_sum;
+        if (gates != nullptr) result = gate_bf16x4(result, gates + out_index + 4 * i);
+        words[2 * i] = pack_bf16x2(result[0], result[1]);
+        words[2 * i + 1] = pack_bf16x2(result[2], result[3]);
+    }
+    if constexpr (QUADS == 2) {
+        *reinterpret_cast<uint4*>(output + out_index) = make_uint4(words[0], words[1], words[2], words[3]);
+    } else {
+        static_assert(QUADS == 1, "one or two quads per lane");
+        *reinterpret_cast<uint2*>(output + out_index) = make_uint2(words[0], words[1]);
+    }
 }
 
 }  // namespace khm

@@ -62,7 +62,7 @@ __global__ __launch_bounds__(kReduceThreads) void split_kv_reduce_kernel(const R
             slice_stats[slice * 2] = state.run_max;
             slice_stats[slice * 2 + 1] = state.run_sum;
         }
-        *reinterpret_cast<f32x4*>(slice_acc + slice * D + chunk * 4) = state.acc;
+        *reinterpret_cast<f32x4*>(slice_acc + slice * D + chunk * 4) = state.acc[0];
         __syncthreads();
         if (slice == 0) {
             const MergeState total = merge_combine_slices<D>(slice_stats, slice_acc, 0, SLICES, chunk);
@@ -72,37 +72,49 @@ __global__ __launch_bounds__(kReduceThreads) void split_kv_reduce_kernel(const R
     }
 }
 
-// The same merge for rows with few partials (speculative-verify tiles have about ten): a group of D/4 threads owns one
-// (token, head) row and walks all of its partials itself, sixteen loads in flight (a row of a decode batch with 512-token
-// partitions has up to sixteen partials), so a block serves 256 / (D/4) rows and nothing passes through LDS.  Rows are numbered (unit * max_q_tokens + token slot) * num_q_heads + head.
-template <int D, bool RANGED>
-__global__ __launch_bounds__(kReduceThreads) void split_kv_reduce_rows_kernel(const ReduceParams p) {
-    constexpr int CHUNKS = D / 4;
-    constexpr int ROWS = kReduceThreads / CHUNKS;
-    const int chunk = threadIdx.x % CHUNKS;
-    const uint64_t row = (uint64_t)blockIdx.x * ROWS + threadIdx.x / CHUNKS;
-    const uint32_t max_q = RANGED ? p.max_q_tokens : 1u;
-    const uint64_t slot = row / p.num_q_heads;
-    const uint32_t head = (uint32_t)(row - slot * p.num_q_heads);
-    const uint32_t unit = (uint32_t)(slot / max_q);
-    const uint32_t local = (uint32_t)(slot - (uint64_t)unit * max_q);
-    if (unit >= resolve_u32(p.num_active, p.replay_parameters)) return;
-    uint32_t flat_begin = unit, num_q = 1;
-    if (RANGED) {
-        flat_begin = p.q_token_ranges[2 * (uint64_t)unit];
-        num_q = p.q_token_ranges[2 * (uint64_t)unit + 1] - flat_begin;
+// The same merge for rows with few partials (speculative-verify tiles have about ten): D/8 threads own one (token, head) row
+// and walk all of its partials themselves, BATCH partials requested at once and 16 bytes per lane, so nothing passes through
+// LDS.  `blocks_per_unit` blocks serve one token (flat) or Q range (ranged), so everything about the unit is block-uniform
+// and read with scalar loads; the live rows of a range are numbered tokens fastest, as the partial states lie in memory: the
+// 4-byte maxima and sums of neighbouring rows share cache lines, and a range with one token of 32 takes blocks for its heads
+// only.  Bound by the bytes of the partial states (which the Map left in the caches).  The batch follows the average number
+// of partials: with sixteen for every row most loads were repeats of a row's first partial.  Before (eight bytes per lane,
+// sixteen requests per row, rows numbered heads first) and now: 1025 tokens of a mixed batch at Hq64/D128 with two to three
+// partials 48.1 -> 20.0 us; 511 tokens at Hq24/D256 with fourteen 26.4 -> 21.3 us; 640 tokens at Hq32/D128 with thirteen
+// 21.5 -> 16.1 us; 61 verify tokens at Hq64/D128 with eight 7.5 -> 5.5 us.  The 16-byte accesses need no more than the
+// 4-byte alignment that global memory instructions ask for.
+template <int D, bool RANGED, int BATCH>
+__global__ __launch_bounds__(kReduceThreads) void split_kv_reduce_rows_kernel(const ReduceParams p, uint32_t blocks_per_unit) {
+    constexpr int OCTETS = D / 8;
+    constexpr int ROWS = kReduceThreads / OCTETS;
+    const uint32_t unit = blockIdx.x / blocks_per_unit;
+    const uint32_t begin = load_uniform_u32(p.cu_partial_outputs, unit);
+    const uint32_t end = load_uniform_u32(p.cu_partial_outputs, (uint64_t)unit + 1);
+    uint32_t flat_begin = unit, num_q = 1, max_q = 1;
+    if constexpr (RANGED) {
+        flat_begin = load_uniform_u32(p.q_token_ranges, 2 * (uint64_t)unit);
+        num_q = load_uniform_u32(p.q_token_ranges, 2 * (uint64_t)unit + 1) - flat_begin;
+        max_q = p.max_q_tokens;
         if (num_q > max_q) num_q = max_q;
     }
-    if (local >= num_q) return;
-    const uint32_t begin = p.cu_partial_outputs[unit];
-    const uint32_t end = p.cu_partial_outputs[unit + 1];
-    MergeState state = merge_state_empty();
-    if (end > begin) {
-        merge_partial_slice<D, false, 16>(state, p.max_logits, p.exp_sums, p.partial, p.partial_is_f32 != 0, begin, end, 1, begin, p.num_q_heads, head,
-                                      max_q, local, chunk);
+    uint32_t active = p.num_active.value;
+    if (p.num_active.is_parameter) active = load_uniform_u32(p.replay_parameters, active);
+    if (unit >= active) return;
+    const uint32_t row = (blockIdx.x - unit * blocks_per_unit) * ROWS + threadIdx.x / OCTETS;
+    if (row >= num_q * p.num_q_heads) return;
+    const int octet = threadIdx.x % OCTETS;
+    const uint32_t head = RANGED ? row / num_q : row;
+    const uint32_t local = RANGED ? row - head * num_q : 0u;
+    const uint64_t row0 = (uint64_t)head * max_q + local, row_step = (uint64_t)p.num_q_heads * max_q;
+    MergeStateOf<2> state = merge_state_empty<2>();
+    if (p.partial_is_f32) {
+        merge_partial_octets<D, true, BATCH / 2>(state, p.max_logits, p.exp_sums, p.partial, begin, end, row0, row_step, octet);
+    } else if (BATCH > 8 && end - begin <= 8) {
+        merge_partial_octets<D, false, 8>(state, p.max_logits, p.exp_sums, p.partial, begin, end, row0, row_step, octet);
+    } else {
+        merge_partial_octets<D, false, BATCH>(state, p.max_logits, p.exp_sums, p.partial, begin, end, row0, row_step, octet);
     }
-    const uint64_t out_index = ((uint64_t)(flat_begin + local) * p.num_q_heads + head) * D + chunk * 4;
-    merge_store_output(state, p.output, p.gates, out_index);
+    merge_store_output(state, p.output, p.gates, ((uint64_t)(flat_begin + local) * p.num_q_heads + head) * D + octet * 8);
 }
 
 // gqa_activation_gate_{f32,bf16} (gqa_activation_gate.metal:28-59): one thread per element.  For buffers that are not

@@ -648,7 +648,7 @@ __global__ __launch_bounds__(NWAVES * 64) void split_kv_map_kernel(const MapPara
                     unit_stats[group * 2] = state.run_max;
                     unit_stats[group * 2 + 1] = state.run_sum;
                 }
-                *reinterpret_cast<f32x4*>(unit_acc + group * D + chunk * 4) = state.acc;
+                *reinterpret_cast<f32x4*>(unit_acc + group * D + chunk * 4) = state.acc[0];
                 __syncthreads();
                 if (live && slice == 0u) state = merge_combine_slices<D>(unit_stats, unit_acc, group, slices, chunk);
             }
