@@ -54,7 +54,7 @@ static TileKernelChoice select_tile_kernel(uint32_t head_dim, uint32_t coordinat
     if (head_dim == 256 && coordinates > 128 && coordinates <= 192) {
         if (kv_dtype == KHM_DTYPE_FP8_E4M3FN) {
             if (direct) return {tile_map_kernel<256, 1, 12, 32, 4, 1, true, true>, 768, (uint32_t)TileSmem<256, 32, 4>::kBytes};
-            return {tile_map_kernel<256, 1, 12, 32, 4, 1, true>, 768, (uint32_t)TileSmem<256, 32, 4>::kBytes};
+            return {tile_map_kernel<256, 1, 12, 32, 4, 1, true>, 768, (uint32_t)TileSmem<256, 32, 4, 256>::kBytes};
         }
         if (direct) return {tile_map_kernel<256, 1, 12, 32, 4, 1, false, true>, 768, (uint32_t)TileSmem<256, 32, 4, 512, true>::kBytes};
         return {tile_map_kernel<256, 1, 12, 32, 4, 1>, 768, (uint32_t)TileSmem<256, 32, 4, 512, true>::kBytes};

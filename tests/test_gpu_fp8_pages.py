@@ -118,3 +118,19 @@ def test_fp8_prefill_other_page_sizes(device, tpp):
     actual = gpu_runner.run_sliced_q(w, ranges, templates, cu, device, kind=sdpa.MAP_Q_TOKENS_AND_HEADS, max_q_tokens=32, max_q_heads=8,
                                      stage=64, direct=True)
     helpers.assert_parity(actual, helpers.expected_output(w), f"fp8 prefill tpp={tpp}")
+
+
+@pytest.mark.parametrize("tpp", [8, 16, 32])
+@pytest.mark.parametrize("kv_slice,partial_dtype", [(33, DTYPE_BF16), (448, DTYPE_F32), (2048, DTYPE_BF16)])
+def test_fp8_twelve_wave_tiles_with_partial_states(device, tpp, kv_slice, partial_dtype):
+    """Tiles of 32 tokens x 6 heads at head dim 256 with partial states: raw codes in LDS shared by twelve waves, eight of which
+    load.  Ranges of one to 32 tokens leave waves without columns, slices start and end off pages and tiles, are shorter than
+    the ring of tiles and longer, and every unused slot of a page holds NaN codes."""
+    histories, q_lens = [0, 61, 700, 3333], [35, 1, 32, 20]
+    w = helpers.make_workload(num_q_heads=12, num_kv_heads=2, head_dim=256, tokens_per_page=tpp, histories=histories, q_lens=q_lens,
+                              seed=500 + tpp, fp8_pages=True, garbage_bits=0x7F)
+    ranges, templates, cu = helpers.fixed_slice_plan(histories, q_lens, 32, kv_slice)
+    print(f"fp8 twelve waves tpp={tpp} kv_slice={kv_slice} partial={partial_dtype}", flush=True)
+    actual = gpu_runner.run_sliced_q(w, ranges, templates, cu, device, kind=sdpa.MAP_Q_TOKENS_AND_HEADS, max_q_tokens=32, max_q_heads=6,
+                                     stage=64, direct=False, partial_dtype=partial_dtype)
+    helpers.assert_parity(actual, helpers.expected_output(w), f"fp8 twelve waves tpp={tpp} slice={kv_slice}")
