@@ -100,18 +100,20 @@ __device__ __forceinline__ void merge_partial_slice(MergeState& state, const flo
     }
 }
 
-// Merges the partials [begin, end) of one row, eight dims per lane (dims octet * 8 .. + 8), BATCH partials requested at once.
+// Merges the partials begin, begin + step, ... < end of one row, eight dims per lane (dims octet * 8 .. + 8), BATCH partials
+// requested at once; `safe_part` is any valid partial index (address of the requests behind the last one).
 // `row0` is the row of partial 0, `row_step` the rows from one partial to the next.
 template <int D, bool F32, int BATCH>
 __device__ __forceinline__ void merge_partial_octets(MergeStateOf<2>& state, const float* max_logits, const float* exp_sums, const void* partial,
-                                                     uint32_t begin, uint32_t end, uint64_t row0, uint64_t row_step, int octet) {
-    for (uint32_t first = begin; first < end; first += BATCH) {
+                                                     uint32_t begin, uint32_t end, uint32_t step, uint32_t safe_part, uint64_t row0, uint64_t row_step, int octet) {
+    for (uint32_t first = begin; first < end; first += BATCH * step) {
         float part_max[BATCH], part_sum[BATCH];
         uint4 bits[BATCH], more[F32 ? BATCH : 1];
 #pragma unroll
         for (int k = 0; k < BATCH; ++k) {
-            const bool ok = first + k < end;
-            const uint64_t row = row0 + (ok ? first + k : begin) * row_step;
+            const uint32_t part = first + k * step;
+            const bool ok = part < end;
+            const uint64_t row = row0 + (ok ? part : safe_part) * row_step;
             part_max[k] = max_logits[row];
             part_sum[k] = ok ? exp_sums[row] : 0.0f;
             const uint4* source = reinterpret_cast<const uint4*>(reinterpret_cast<const unsigned char*>(partial) + (row * D + octet * 8) * (F32 ? 4 : 2));
@@ -151,15 +153,30 @@ __device__ __forceinline__ MergeState merge_combine_slices(const float* stats, c
     return out;
 }
 
+// The gate values of a lane's dims.  Nothing that the merge computes decides where they are, so they are requested first.
+template <int QUADS>
+struct GateBits {
+    uint2 quad[QUADS];
+    bool gated;
+};
+template <int QUADS = 1>
+__device__ __forceinline__ GateBits<QUADS> request_gates(const uint16_t* gates, uint64_t out_index) {
+    GateBits<QUADS> bits;
+    bits.gated = gates != nullptr;
+#pragma unroll
+    for (int i = 0; i < QUADS; ++i) bits.quad[i] = bits.gated ? *reinterpret_cast<const uint2*>(gates + out_index + 4 * i) : make_uint2(0, 0);
+    return bits;
+}
+
 // Normalizes, applies the optional bf16 gate (gqa_activation_gate.metal:19-39) and stores four bf16 outputs per quad.
 template <int QUADS>
-__device__ __forceinline__ void merge_store_output(const MergeStateOf<QUADS>& state, uint16_t* output, const uint16_t* gates, uint64_t out_index) {
+__device__ __forceinline__ void merge_store_output(const MergeStateOf<QUADS>& state, uint16_t* output, const GateBits<QUADS>& gates, uint64_t out_index) {
     uint32_t words[2 * QUADS];
 #pragma unroll
     for (int i = 0; i < QUADS; ++i) {
         f32x4 result = {0.0f, 0.0f, 0.0f, 0.0f};
         if (state.run_sum > 0.0f) result = state.acc[i] / state.run_sum;
-        if (gates != nullptr) result = gate_bf16x4(result, gates + out_index + 4 * i);
+        if (gates.gated) result = gate_bf16x4(result, gates.quad[i]);
         words[2 * i] = pack_bf16x2(result[0], result[1]);
         words[2 * i + 1] = pack_bf16x2(result[2], result[3]);
     }

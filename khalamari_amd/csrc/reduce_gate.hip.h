@@ -5,8 +5,8 @@
 // gqa_sdpa_sliced_q_reduce (.../gqa_sdpa_sliced_q_reduce.metal:4-63):
 //     gmax = max_p max_p;  w_p = exp(max_p - gmax) * sum_p  (0 for an empty partial);
 //     out  = sum_p w_p * partial_p / sum_p w_p              (0 when the denominator is 0)
-// One block owns one output row group; its threads are arranged as
-// (partial-slice, 4-dim chunk): every slice walks a strided subset of the row's partials with
+// One block owns one output row; its threads are arranged as
+// (partial-slice, 8-dim octet): every slice walks a strided subset of the row's partials with
 // its own running maximum, and the slices are merged through LDS.  Long rows (a 131072-token
 // context has 64 partials at 2048-token partitions) therefore reduce in parallel instead of in
 // one thread's serial loop.
@@ -28,48 +28,57 @@ constexpr int kReduceThreads = 256;
 // RANGED = false: sliced-KV flat reduce, grid (tokens, heads).
 // RANGED = true : sliced-Q reduce, grid (Q ranges * max_q_tokens, heads): one block per token slot of a range, so the
 //                 tokens of a range reduce side by side rather than in a serial loop of dependent loads.
+// Few rows with many partials: bound by the round trips to memory one after the other.  D/8 threads of 16 bytes share a
+// partial, so a block has eight (D 256) or sixteen slices of the list and 64 partials are requested at once, with the gate
+// values (four 131072-token contexts at Hq24/D256, 64
+// partials a row: 7.3 us with 8-byte loads, four slices and two batches each, 5.2 us now).
 template <int D, bool RANGED>
 __global__ __launch_bounds__(kReduceThreads) void split_kv_reduce_kernel(const ReduceParams p) {
-    constexpr int CHUNKS = D / 4;                    // threads per row
-    constexpr int SLICES = kReduceThreads / CHUNKS;  // partial slices per block
+    constexpr int OCTETS = D / 8;                    // threads per partial
+    constexpr int SLICES = kReduceThreads / OCTETS;  // partial slices per block
+    constexpr int BATCH = 64 / SLICES;
     __shared__ float slice_stats[SLICES * 2];
     __shared__ __align__(16) float slice_acc[SLICES * D];
 
     const uint32_t unit = RANGED ? blockIdx.x / p.max_q_tokens : blockIdx.x;
-    if (unit >= resolve_u32(p.num_active, p.replay_parameters)) return;
     const uint32_t head = blockIdx.y;
-    const uint32_t begin = p.cu_partial_outputs[unit];
-    const uint32_t end = p.cu_partial_outputs[unit + 1];
+    const uint32_t begin = load_uniform_u32(p.cu_partial_outputs, unit);
+    const uint32_t end = load_uniform_u32(p.cu_partial_outputs, (uint64_t)unit + 1);
     uint32_t flat_begin = unit, num_q = 1, max_q = 1;
-    if (RANGED) {
-        flat_begin = p.q_token_ranges[2 * (uint64_t)unit];
-        num_q = p.q_token_ranges[2 * (uint64_t)unit + 1] - flat_begin;
+    if constexpr (RANGED) {
+        flat_begin = load_uniform_u32(p.q_token_ranges, 2 * (uint64_t)unit);
+        num_q = load_uniform_u32(p.q_token_ranges, 2 * (uint64_t)unit + 1) - flat_begin;
         max_q = p.max_q_tokens;
         if (num_q > max_q) num_q = max_q;
     }
-    const int chunk = threadIdx.x % CHUNKS;
-    const uint32_t slice = threadIdx.x / CHUNKS;
-
+    uint32_t active = p.num_active.value;
+    if (p.num_active.is_parameter) active = load_uniform_u32(p.replay_parameters, active);
+    if (unit >= active) return;
     const uint32_t local = RANGED ? blockIdx.x - unit * p.max_q_tokens : 0u;
     if (local >= num_q) return;
-    {
-        MergeState state = merge_state_empty();
-        if (end > begin) {
-            merge_partial_slice<D, false>(state, p.max_logits, p.exp_sums, p.partial, p.partial_is_f32 != 0, begin + slice, end, SLICES, begin,
-                                          p.num_q_heads, head, max_q, local, chunk);
-        }
-        if (chunk == 0) {
-            slice_stats[slice * 2] = state.run_max;
-            slice_stats[slice * 2 + 1] = state.run_sum;
-        }
-        *reinterpret_cast<f32x4*>(slice_acc + slice * D + chunk * 4) = state.acc[0];
-        __syncthreads();
-        if (slice == 0) {
-            const MergeState total = merge_combine_slices<D>(slice_stats, slice_acc, 0, SLICES, chunk);
-            const uint64_t out_index = ((uint64_t)(flat_begin + local) * p.num_q_heads + head) * D + chunk * 4;
-            merge_store_output(total, p.output, p.gates, out_index);
-        }
+
+    const int octet = threadIdx.x % OCTETS;
+    const uint32_t slice = threadIdx.x / OCTETS;
+    // the first D/4 threads write four dims each
+    const uint64_t out_index = ((uint64_t)(flat_begin + local) * p.num_q_heads + head) * D + threadIdx.x * 4;
+    const bool writes = threadIdx.x < D / 4;
+    const GateBits<1> gates = request_gates(writes ? p.gates : nullptr, out_index);
+    const uint64_t row0 = (uint64_t)head * max_q + local, row_step = (uint64_t)p.num_q_heads * max_q;
+    MergeStateOf<2> state = merge_state_empty<2>();
+    if (end > begin) {
+        if (p.partial_is_f32)
+            merge_partial_octets<D, true, BATCH>(state, p.max_logits, p.exp_sums, p.partial, begin + slice, end, SLICES, begin, row0, row_step, octet);
+        else
+            merge_partial_octets<D, false, BATCH>(state, p.max_logits, p.exp_sums, p.partial, begin + slice, end, SLICES, begin, row0, row_step, octet);
     }
+    if (octet == 0) {
+        slice_stats[slice * 2] = state.run_max;
+        slice_stats[slice * 2 + 1] = state.run_sum;
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) *reinterpret_cast<f32x4*>(slice_acc + slice * D + octet * 8 + i * 4) = state.acc[i];
+    __syncthreads();
+    if (writes) merge_store_output(merge_combine_slices<D>(slice_stats, slice_acc, 0, SLICES, threadIdx.x), p.output, gates, out_index);
 }
 
 // The same merge for rows with few partials (speculative-verify tiles have about ten): D/8 threads own one (token, head) row
@@ -106,15 +115,17 @@ __global__ __launch_bounds__(kReduceThreads) void split_kv_reduce_rows_kernel(co
     const uint32_t head = RANGED ? row / num_q : row;
     const uint32_t local = RANGED ? row - head * num_q : 0u;
     const uint64_t row0 = (uint64_t)head * max_q + local, row_step = (uint64_t)p.num_q_heads * max_q;
+    const uint64_t out_index = ((uint64_t)(flat_begin + local) * p.num_q_heads + head) * D + octet * 8;
+    const GateBits<2> gates = request_gates<2>(p.gates, out_index);
     MergeStateOf<2> state = merge_state_empty<2>();
     if (p.partial_is_f32) {
-        merge_partial_octets<D, true, BATCH / 2>(state, p.max_logits, p.exp_sums, p.partial, begin, end, row0, row_step, octet);
+        merge_partial_octets<D, true, BATCH / 2>(state, p.max_logits, p.exp_sums, p.partial, begin, end, 1, begin, row0, row_step, octet);
     } else if (BATCH > 8 && end - begin <= 8) {
-        merge_partial_octets<D, false, 8>(state, p.max_logits, p.exp_sums, p.partial, begin, end, row0, row_step, octet);
+        merge_partial_octets<D, false, 8>(state, p.max_logits, p.exp_sums, p.partial, begin, end, 1, begin, row0, row_step, octet);
     } else {
-        merge_partial_octets<D, false, BATCH>(state, p.max_logits, p.exp_sums, p.partial, begin, end, row0, row_step, octet);
+        merge_partial_octets<D, false, BATCH>(state, p.max_logits, p.exp_sums, p.partial, begin, end, 1, begin, row0, row_step, octet);
     }
-    merge_store_output(state, p.output, p.gates, ((uint64_t)(flat_begin + local) * p.num_q_heads + head) * D + octet * 8);
+    merge_store_output(state, p.output, gates, out_index);
 }
 
 // gqa_activation_gate_{f32,bf16} (gqa_activation_gate.metal:28-59): one thread per element.  For buffers that are not

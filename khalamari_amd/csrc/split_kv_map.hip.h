@@ -654,7 +654,7 @@ __global__ __launch_bounds__(NWAVES * 64) void split_kv_map_kernel(const MapPara
             }
             if (live && slice == 0u) {
                 const uint64_t out_index = ((uint64_t)(flat_begin + token_offset) * p.num_q_heads + q_head) * D + chunk * 4;
-                merge_store_output(state, p.final_output, p.gates, out_index);
+                merge_store_output(state, p.final_output, request_gates(p.gates, out_index), out_index);
             }
             if (slices > 1u) __syncthreads();
         }
