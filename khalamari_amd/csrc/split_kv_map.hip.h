@@ -67,7 +67,7 @@ struct MapSmem {
 constexpr int kMapPrefetchDepth = 2;
 
 template <int D, int NT, int NWAVES, bool KV8 = false>
-__global__ __launch_bounds__(NWAVES * 64) void split_kv_map_kernel(const MapParams p) {
+__global__ __launch_bounds__(NWAVES * 64, (KV8 && D == 128) ? 4 : 1) void split_kv_map_kernel(const MapParams p) {
     constexpr int KS = D / 32;
     constexpr int MT = D / 16;
     constexpr int COLS = NT * 16;
@@ -83,8 +83,13 @@ __global__ __launch_bounds__(NWAVES * 64) void split_kv_map_kernel(const MapPara
     // run at the pace of their own load -> decode -> MFMA chain, which a second wave on the SIMD overlaps (four requests of
     // 131072 tokens: 200 -> 194 us).  bf16 pages at D 256 stay at one block either way (399 registers) and are within 3 %
     // of a read-only launch; at D 128 a third block per CU was measured and changes nothing.
+    // D 128 on FP8 pages: with Q in LDS and the accumulator in ordinary registers (128 of them, 36 AGPRs beside them before) a
+    // compute unit holds four blocks instead of three, which a grid of 1024 equal blocks fills in one round instead of one and
+    // a third: 45 requests of 300..12000 tokens at Hq64/Hkv8 layer 119.4 -> 112.2 us, 60 of 511..8000 at Hq32/Hkv8 123.8 ->
+    // 115.1 us; four of 131072 in 2048 blocks 194.6 -> 196.0 us.
     constexpr bool kSlim = D == 256 && KV8;
-    constexpr bool kQInRegs = (NT == 1) && !kSlim;
+    constexpr bool kFourBlocks = D == 128 && KV8;
+    constexpr bool kQInRegs = (NT == 1) && !kSlim && !kFourBlocks;
     using Smem = MapSmem<D, NT, NWAVES, !kQInRegs>;
 
     __shared__ __align__(16) unsigned char smem[Smem::kTotal];
@@ -372,7 +377,7 @@ __global__ __launch_bounds__(NWAVES * 64) void split_kv_map_kernel(const MapPara
                 run_sum[nt] *= alpha;
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt) {
-                    asm volatile("" : "+a"(acc[nt][mt]));   // the move out of the AGPRs belongs to this branch
+                    if constexpr (!kFourBlocks) asm volatile("" : "+a"(acc[nt][mt]));   // the move out of the AGPRs belongs to this branch
                     acc[nt][mt] *= alpha;
                 }
             }
@@ -438,12 +443,14 @@ __global__ __launch_bounds__(NWAVES * 64) void split_kv_map_kernel(const MapPara
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
+        // (Not with four blocks per CU, where the wave has 128 registers in all.)
         // The accumulator stays in the AGPR half of the register file from tile to tile (only the rare rescale moves
         // it through VGPRs); without the pin the compiler keeps a second copy in VGPRs and refreshes it after every tile.
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-            for (int mt = 0; mt < MT; ++mt) asm volatile("" : "+a"(acc[nt][mt]));
+            for (int mt = 0; mt < MT; ++mt)
+                if constexpr (!kFourBlocks) asm volatile("" : "+a"(acc[nt][mt]));
     };
 
     // ---- main loop: a ring of register buffers, loads DEPTH tiles ahead ----------------------
