@@ -66,8 +66,19 @@ struct MapSmem {
 // K/V tiles requested ahead of the one being consumed (register buffers: one more than this).
 constexpr int kMapPrefetchDepth = 2;
 
-template <int D, int NT, int NWAVES, bool KV8 = false>
-__global__ __launch_bounds__(NWAVES * 64, (KV8 && D == 128) ? 4 : 1) void split_kv_map_kernel(const MapParams p) {
+// Bytes of LDS a block works in.
+template <int D, int NT, int NWAVES, bool KV8>
+constexpr int split_kv_map_smem_bytes() { return MapSmem<D, NT, NWAVES, NT != 1 || KV8>::kTotal; }
+
+// What a block knows about its task; everything is block-uniform.
+struct MapTask {
+    uint32_t task, head_group, range_index, kv_begin, kv_end, flat_begin, num_q, req_slot, layer, num_active_splits;
+};
+
+// One block's work.  `smem` holds split_kv_map_smem_bytes.  ACC_IN_AGPRS: the accumulator is held in the AGPR half of the
+// register file (see the end of compute_tile); CAN_MERGE: the call may ask for the Reduce in the last block.
+template <int D, int NT, int NWAVES, bool KV8, bool ACC_IN_AGPRS, bool CAN_MERGE>
+__device__ __forceinline__ void split_kv_map_block(const MapParams& p, const MapTask& t, unsigned char* smem) {
     constexpr int KS = D / 32;
     constexpr int MT = D / 16;
     constexpr int COLS = NT * 16;
@@ -92,7 +103,6 @@ __global__ __launch_bounds__(NWAVES * 64, (KV8 && D == 128) ? 4 : 1) void split_
     constexpr bool kQInRegs = (NT == 1) && !kSlim && !kFourBlocks;
     using Smem = MapSmem<D, NT, NWAVES, !kQInRegs>;
 
-    __shared__ __align__(16) unsigned char smem[Smem::kTotal];
     unsigned char* v_lds_all = smem;
     float* o_lds = reinterpret_cast<float*>(smem);
     unsigned char* q_lds = smem + Smem::kUnionBytes;
@@ -104,40 +114,8 @@ __global__ __launch_bounds__(NWAVES * 64, (KV8 && D == 128) ? 4 : 1) void split_
     const int r16 = lane & 15;
     const int g = lane >> 4;
 
-    // ---- task decode (uniform) -------------------------------------------------------------
-    // Blocks are dispatched in linear order; the KV heads of one task vary fastest, so the blocks in flight together
-    // read neighbouring slabs of the same pages (a whole 64 KB page between the eight heads) instead of the same
-    // 4 KB window of many pages, which spreads the requests evenly over the memory channels (+4 % on config 2).
-    const uint32_t linear_block = blockIdx.y * gridDim.x + blockIdx.x;
-    const uint32_t task = linear_block / gridDim.y;
-    const uint32_t head_group_index = linear_block % gridDim.y;
-    // The metadata chain in front of a block's first K/V load is a chain of dependent round trips to memory, a fifth of
-    // the life of a 512-token decode block: arguments -> task template -> request slot -> page ids -> K/V.  Every link is
-    // a scalar load, and everything that hangs on the same link is requested together: the whole argument block; then
-    // the template's three words and the replay values; then (sliced-Q) the Q range; then the request slot.  The grid
-    // has one block per template of the padded shape, so reading the template before the activity test is in bounds.
-    fetch_all_arguments(p);
-    const ReplayValues replay = resolve_replay_values(p);
-    const uint32_t range_index = load_uniform_u32(p.templates, 3 * (uint64_t)task);
-    const uint32_t kv_begin = load_uniform_u32(p.templates, 3 * (uint64_t)task + 1);
-    const uint32_t kv_end = load_uniform_u32(p.templates, 3 * (uint64_t)task + 2);
-    const uint32_t num_active_splits = replay.num_active_kv_splits;
-    if (task >= num_active_splits) return;
-    if (range_index >= replay.num_active_q_token_tiles) return;
-    uint32_t flat_begin, flat_end;
-    if (p.q_token_ranges != nullptr) {
-        flat_begin = load_uniform_u32(p.q_token_ranges, 2 * (uint64_t)range_index);
-        flat_end = load_uniform_u32(p.q_token_ranges, 2 * (uint64_t)range_index + 1);
-    } else {
-        flat_begin = range_index;
-        flat_end = range_index + 1;
-    }
-    const uint32_t num_active_tokens = replay.num_active_tokens;
-    if (flat_begin >= num_active_tokens || flat_end > num_active_tokens || flat_end <= flat_begin) return;
-    uint32_t num_q = flat_end - flat_begin;
-    if (num_q > p.max_q_tokens) num_q = p.max_q_tokens;
-    const uint32_t req_slot = load_uniform_u32(p.req_slots, flat_begin);
-    const uint32_t layer = replay.layer;
+    const uint32_t task = t.task, head_group_index = t.head_group, range_index = t.range_index, kv_begin = t.kv_begin, kv_end = t.kv_end;
+    const uint32_t flat_begin = t.flat_begin, num_q = t.num_q, req_slot = t.req_slot, layer = t.layer, num_active_splits = t.num_active_splits;
 
     const uint32_t head_range = head_group_index % p.num_q_head_ranges;
     const uint32_t kv_head = head_group_index / p.num_q_head_ranges;
@@ -377,7 +355,7 @@ __global__ __launch_bounds__(NWAVES * 64, (KV8 && D == 128) ? 4 : 1) void split_
                 run_sum[nt] *= alpha;
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt) {
-                    if constexpr (!kFourBlocks) asm volatile("" : "+a"(acc[nt][mt]));   // the move out of the AGPRs belongs to this branch
+                    if constexpr (ACC_IN_AGPRS) asm volatile("" : "+a"(acc[nt][mt]));   // the move out of the AGPRs belongs to this branch
                     acc[nt][mt] *= alpha;
                 }
             }
@@ -450,7 +428,7 @@ __global__ __launch_bounds__(NWAVES * 64, (KV8 && D == 128) ? 4 : 1) void split_
         for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt)
-                if constexpr (!kFourBlocks) asm volatile("" : "+a"(acc[nt][mt]));
+                if constexpr (ACC_IN_AGPRS) asm volatile("" : "+a"(acc[nt][mt]));
     };
 
     // ---- main loop: a ring of register buffers, loads DEPTH tiles ahead ----------------------
@@ -543,7 +521,7 @@ __global__ __launch_bounds__(NWAVES * 64, (KV8 && D == 128) ? 4 : 1) void split_
 
     // ---- write the block's partial state or final output ------------------------------------
     const uint32_t mode = p.output_mode;
-    const bool fused = p.arrival_counters != nullptr && mode != kMapDirectBf16;
+    const bool fused = CAN_MERGE && p.arrival_counters != nullptr && mode != kMapDirectBf16;
     for (int index = tid; index < COLS * (D / 4); index += NWAVES * 64) {
         const uint32_t c = index / (D / 4);
         const uint32_t d = (index - c * (D / 4)) * 4;
@@ -598,74 +576,116 @@ __global__ __launch_bounds__(NWAVES * 64, (KV8 && D == 128) ? 4 : 1) void split_
     }
 
     // ---- fused Reduce: the last block of a (Q range, head group) merges all of its partial states ----------
-    if (!fused) return;
-    // Publishing the partial state to whichever block merges it.  Every store above is a device-coherent (sc1,
-    // write-through) store: it is never held dirty in this XCD's L2, so what a release needs here is only that each wave
-    // waits until its own stores have been acknowledged - the explicit wait below, which does not depend on what the
-    // compiler puts in front of a barrier.  (A release fence at agent scope adds an L2 write-back per wave with nothing to
-    // write back, and that alone takes a 2272-block launch from 114 to 209 us.)  The barrier then orders all waves' stores
-    // before thread 0 signals arrival; the arrival is an acquire, so the block that sees the last one reads the others'
-    // partial states - through device-coherent loads - after their stores.
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    uint32_t* flag_lds = reinterpret_cast<uint32_t*>(stats_lds);
-    const uint32_t partial_begin = p.cu_partial_outputs[range_index];
-    uint32_t partial_end = p.cu_partial_outputs[range_index + 1];
-    if (partial_end > num_active_splits) partial_end = num_active_splits;
-    if (tid == 0) {
-        uint32_t* counter = p.arrival_counters + (uint64_t)range_index * gridDim.y + head_group_index;
-        const uint32_t arrived = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT) + 1u;
-        const uint32_t last = arrived == partial_end - partial_begin ? 1u : 0u;
-        if (last) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // re-arm for the next launch
-        flag_lds[0] = last;
-    }
-    __syncthreads();
-    if (flag_lds[0] == 0u) return;
-    {
-        // Work units are (column, partial-slice) pairs; a group of D/4 lanes owns one unit at a time and walks
-        // its partials with an online merge, eight partials' loads in flight at once.  With at least as many
-        // columns as groups every column has one slice and a group writes its column's output directly;
-        // with fewer columns the spare groups split the partial list and combine through LDS.
-        constexpr int CHUNKS = D / 4;
-        constexpr int GROUPS = NWAVES * 64 / CHUNKS;
-        const int chunk = tid % CHUNKS;
-        const uint32_t group = tid / CHUNKS;
-        const uint32_t active_cols = num_q * p.max_q_heads;
-        const uint32_t slices = active_cols >= (uint32_t)GROUPS ? 1u : (uint32_t)GROUPS / active_cols;
-        const uint32_t num_units = active_cols * slices;
-        float* unit_acc = o_lds;                 // [GROUPS][D]
-        float* unit_stats = o_lds + GROUPS * D;  // [GROUPS][2]
-        const bool f32_partials = mode == kMapPartialF32;
-        for (uint32_t base = 0; base < num_units; base += GROUPS) {
-            const uint32_t unit = base + group;
-            const bool has_unit = unit < num_units;
-            const uint32_t c = has_unit ? unit / slices : 0u;
-            const uint32_t slice = unit - c * slices;
-            const uint32_t token_offset = c / p.max_q_heads;
-            const uint32_t local_head = c - token_offset * p.max_q_heads;
-            const bool live = has_unit && local_head < num_heads;
-            const uint32_t q_head = first_q_head + (live ? local_head : 0u);
-            MergeState state = merge_state_empty();
-            if (live) {
-                merge_partial_slice<D, true>(state, p.max_logits, p.exp_sums, p.out, f32_partials, partial_begin + slice, partial_end, slices,
-                                             partial_begin, p.num_q_heads, q_head, p.max_q_tokens, token_offset, chunk);
-            }
-            if (slices > 1u) {
-                if (chunk == 0) {
-                    unit_stats[group * 2] = state.run_max;
-                    unit_stats[group * 2 + 1] = state.run_sum;
+    if constexpr (CAN_MERGE) {
+        if (!fused) return;
+        // Publishing the partial state to whichever block merges it.  Every store above is a device-coherent (sc1,
+        // write-through) store: it is never held dirty in this XCD's L2, so what a release needs here is only that each wave
+        // waits until its own stores have been acknowledged - the explicit wait below, which does not depend on what the
+        // compiler puts in front of a barrier.  (A release fence at agent scope adds an L2 write-back per wave with nothing to
+        // write back, and that alone takes a 2272-block launch from 114 to 209 us.)  The barrier then orders all waves' stores
+        // before thread 0 signals arrival; the arrival is an acquire, so the block that sees the last one reads the others'
+        // partial states - through device-coherent loads - after their stores.
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        uint32_t* flag_lds = reinterpret_cast<uint32_t*>(stats_lds);
+        const uint32_t partial_begin = p.cu_partial_outputs[range_index];
+        uint32_t partial_end = p.cu_partial_outputs[range_index + 1];
+        if (partial_end > num_active_splits) partial_end = num_active_splits;
+        if (tid == 0) {
+            uint32_t* counter = p.arrival_counters + (uint64_t)range_index * gridDim.y + head_group_index;
+            const uint32_t arrived = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT) + 1u;
+            const uint32_t last = arrived == partial_end - partial_begin ? 1u : 0u;
+            if (last) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // re-arm for the next launch
+            flag_lds[0] = last;
+        }
+        __syncthreads();
+        if (flag_lds[0] == 0u) return;
+        {
+            // Work units are (column, partial-slice) pairs; a group of D/4 lanes owns one unit at a time and walks
+            // its partials with an online merge, eight partials' loads in flight at once.  With at least as many
+            // columns as groups every column has one slice and a group writes its column's output directly;
+            // with fewer columns the spare groups split the partial list and combine through LDS.
+            constexpr int CHUNKS = D / 4;
+            constexpr int GROUPS = NWAVES * 64 / CHUNKS;
+            const int chunk = tid % CHUNKS;
+            const uint32_t group = tid / CHUNKS;
+            const uint32_t active_cols = num_q * p.max_q_heads;
+            const uint32_t slices = active_cols >= (uint32_t)GROUPS ? 1u : (uint32_t)GROUPS / active_cols;
+            const uint32_t num_units = active_cols * slices;
+            float* unit_acc = o_lds;                 // [GROUPS][D]
+            float* unit_stats = o_lds + GROUPS * D;  // [GROUPS][2]
+            const bool f32_partials = mode == kMapPartialF32;
+            for (uint32_t base = 0; base < num_units; base += GROUPS) {
+                const uint32_t unit = base + group;
+                const bool has_unit = unit < num_units;
+                const uint32_t c = has_unit ? unit / slices : 0u;
+                const uint32_t slice = unit - c * slices;
+                const uint32_t token_offset = c / p.max_q_heads;
+                const uint32_t local_head = c - token_offset * p.max_q_heads;
+                const bool live = has_unit && local_head < num_heads;
+                const uint32_t q_head = first_q_head + (live ? local_head : 0u);
+                MergeState state = merge_state_empty();
+                if (live) {
+                    merge_partial_slice<D, true>(state, p.max_logits, p.exp_sums, p.out, f32_partials, partial_begin + slice, partial_end, slices,
+                                                 partial_begin, p.num_q_heads, q_head, p.max_q_tokens, token_offset, chunk);
                 }
-                *reinterpret_cast<f32x4*>(unit_acc + group * D + chunk * 4) = state.acc[0];
-                __syncthreads();
-                if (live && slice == 0u) state = merge_combine_slices<D>(unit_stats, unit_acc, group, slices, chunk);
+                if (slices > 1u) {
+                    if (chunk == 0) {
+                        unit_stats[group * 2] = state.run_max;
+                        unit_stats[group * 2 + 1] = state.run_sum;
+                    }
+                    *reinterpret_cast<f32x4*>(unit_acc + group * D + chunk * 4) = state.acc[0];
+                    __syncthreads();
+                    if (live && slice == 0u) state = merge_combine_slices<D>(unit_stats, unit_acc, group, slices, chunk);
+                }
+                if (live && slice == 0u) {
+                    const uint64_t out_index = ((uint64_t)(flat_begin + token_offset) * p.num_q_heads + q_head) * D + chunk * 4;
+                    merge_store_output(state, p.final_output, request_gates(p.gates, out_index), out_index);
+                }
+                if (slices > 1u) __syncthreads();
             }
-            if (live && slice == 0u) {
-                const uint64_t out_index = ((uint64_t)(flat_begin + token_offset) * p.num_q_heads + q_head) * D + chunk * 4;
-                merge_store_output(state, p.final_output, request_gates(p.gates, out_index), out_index);
-            }
-            if (slices > 1u) __syncthreads();
         }
     }
+}
+
+template <int D, int NT, int NWAVES, bool KV8 = false>
+__global__ __launch_bounds__(NWAVES * 64, (KV8 && D == 128) ? 4 : 1) void split_kv_map_kernel(const MapParams p) {
+    __shared__ __align__(16) unsigned char smem[split_kv_map_smem_bytes<D, NT, NWAVES, KV8>()];
+    // ---- task decode (uniform) -------------------------------------------------------------
+    // Blocks are dispatched in linear order; the KV heads of one task vary fastest, so the blocks in flight together
+    // read neighbouring slabs of the same pages (a whole 64 KB page between the eight heads) instead of the same
+    // 4 KB window of many pages, which spreads the requests evenly over the memory channels (+4 % on config 2).
+    const uint32_t linear_block = blockIdx.y * gridDim.x + blockIdx.x;
+    const uint32_t task = linear_block / gridDim.y;
+    const uint32_t head_group_index = linear_block % gridDim.y;
+    // The metadata chain in front of a block's first K/V load is a chain of dependent round trips to memory, a fifth of
+    // the life of a 512-token decode block: arguments -> task template -> request slot -> page ids -> K/V.  Every link is
+    // a scalar load, and everything that hangs on the same link is requested together: the whole argument block; then
+    // the template's three words and the replay values; then (sliced-Q) the Q range; then the request slot.  The grid
+    // has one block per template of the padded shape, so reading the template before the activity test is in bounds.
+    fetch_all_arguments(p);
+    const ReplayValues replay = resolve_replay_values(p);
+    const uint32_t range_index = load_uniform_u32(p.templates, 3 * (uint64_t)task);
+    const uint32_t kv_begin = load_uniform_u32(p.templates, 3 * (uint64_t)task + 1);
+    const uint32_t kv_end = load_uniform_u32(p.templates, 3 * (uint64_t)task + 2);
+    const uint32_t num_active_splits = replay.num_active_kv_splits;
+    if (task >= num_active_splits) return;
+    if (range_index >= replay.num_active_q_token_tiles) return;
+    uint32_t flat_begin, flat_end;
+    if (p.q_token_ranges != nullptr) {
+        flat_begin = load_uniform_u32(p.q_token_ranges, 2 * (uint64_t)range_index);
+        flat_end = load_uniform_u32(p.q_token_ranges, 2 * (uint64_t)range_index + 1);
+    } else {
+        flat_begin = range_index;
+        flat_end = range_index + 1;
+    }
+    const uint32_t num_active_tokens = replay.num_active_tokens;
+    if (flat_begin >= num_active_tokens || flat_end > num_active_tokens || flat_end <= flat_begin) return;
+    uint32_t num_q = flat_end - flat_begin;
+    if (num_q > p.max_q_tokens) num_q = p.max_q_tokens;
+    const uint32_t req_slot = load_uniform_u32(p.req_slots, flat_begin);
+    const uint32_t layer = replay.layer;
+    split_kv_map_block<D, NT, NWAVES, KV8, !(KV8 && D == 128), true>(p, MapTask{task, head_group_index, range_index, kv_begin, kv_end, flat_begin, num_q, req_slot, layer, num_active_splits}, smem);
 }
 
 }  // namespace khm

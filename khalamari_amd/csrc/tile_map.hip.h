@@ -27,6 +27,7 @@
 #include "device_math.hip.h"
 #include "device_params.h"
 #include "fp8_device.hip.h"
+#include "split_kv_map.hip.h"
 
 namespace khm {
 
@@ -211,6 +212,18 @@ void tile_map_kernel(const MapParams p) {
     if (num_q > p.max_q_tokens) num_q = p.max_q_tokens;
     const uint32_t req_slot = load_uniform_u32(p.req_slots, flat_begin);
     const uint32_t layer = replay.layer;
+    if constexpr (D == 128 && NTW == 2) {
+        // A range that fills one column tile or less (a request that decodes beside others that run a chunk) leaves all waves but
+        // one without columns; the waves share its tokens instead, as in the decode kernel, whose accumulator fits beside
+        // the wide path's registers at head dim 128.  Hq64/Hkv8 on FP8 pages: 25 such requests beside two 500-token chunks,
+        // layer 236.2 -> 220.0 us; 59 of 1000..16000 tokens beside one chunk of 100 389 -> 225 us; bf16 pages 229.4 -> 222.8 us.
+        // Four waves, Hq32/Hkv8: 199.9 -> 179.3 and 436 -> 287 us (2048-token chunks without such ranges 3.776 -> 3.799 ms).
+        static_assert(split_kv_map_smem_bytes<D, 1, NWAVES, KV8>() <= Smem::kBytes, "the block's LDS holds the decode kernel's");
+        if (num_q * p.max_q_heads <= 16) {
+            split_kv_map_block<D, 1, NWAVES, KV8, false, false>(p, MapTask{task, head_group, range_index, kv_begin, kv_end, flat_begin, num_q, req_slot, layer, replay.num_active_kv_splits}, tile_smem);
+            return;
+        }
+    }
 
     const uint32_t head_range = head_group % p.num_q_head_ranges;
     const uint32_t kv_head = head_group / p.num_q_head_ranges;

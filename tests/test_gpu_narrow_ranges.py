@@ -1,0 +1,26 @@
+"""Q ranges that fill at most one 16-column tile beside wide ones in the same launch (requests that decode beside a chunk): the waves
+of a block share such a range's tokens.  Ranges on both sides of the line, slices off every boundary, NaN in unused slots."""
+import pytest
+
+from khalamari_amd import sdpa
+from khalamari_amd._lib import DTYPE_BF16, DTYPE_F32
+
+from . import gpu_runner, helpers
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("hq,hkv,tpp", [(64, 8, 16), (10, 2, 8), (16, 1, 16), (8, 2, 16)])
+def test_narrow_ranges_beside_wide_ones(device, hq, hkv, tpp, fp8):
+    histories, q_lens = [0, 2100, 5, 700, 130, 16, 64, 1023], [1, 1, 2, 33, 3, 4, 5, 1]
+    ratio, tile = hq // hkv, 32 if hq // hkv <= 8 else 16
+    w = helpers.make_workload(num_q_heads=hq, num_kv_heads=hkv, head_dim=128, tokens_per_page=tpp, histories=histories, q_lens=q_lens,
+                              seed=hq + tpp, fp8_pages=fp8, garbage_bits=0x7F if fp8 else 0x7FC0)
+    expected = helpers.expected_output(w)
+    for kv_slice, direct, partial in [(1 << 20, True, DTYPE_BF16), (333, False, DTYPE_BF16), (64, False, DTYPE_F32)]:
+        ranges, templates, cu = helpers.fixed_slice_plan(histories, q_lens, tile, kv_slice)
+        print(f"narrow ranges Hq{hq}/Hkv{hkv} tpp={tpp} fp8={fp8} slice={kv_slice} direct={direct}", flush=True)
+        common = dict(kind=sdpa.MAP_Q_TOKENS_AND_HEADS, max_q_tokens=tile, max_q_heads=ratio, stage=64, direct=direct, partial_dtype=partial)
+        actual = gpu_runner.run_sliced_q(w, ranges, templates, cu, device, **common)
+        helpers.assert_parity(actual, expected, f"narrow ranges slice={kv_slice} direct={direct}")
