@@ -6,7 +6,7 @@ import ctypes
 from dataclasses import dataclass
 
 from . import _lib
-from ._buffers import param_block, stream_handle, view
+from ._buffers import pack, param_block, stream_handle
 from ._lib import DTYPE_BF16, DTYPE_F32, BidiBlockSdpaBuffers, BidiBlockSdpaConfig, BidiBlockSdpaShape, ReplayU32
 
 
@@ -56,7 +56,7 @@ class Compute:
     def invoke(self, shape: Shape, num_active_q_token_ranges: ReplayU32, *, q, local_k, local_v, q_token_ranges, cu_sdpa_partial_outputs,
                partial_exp_sums, partial_max_logits, partial_output, replay_parameters=None, stream=None) -> None:
         config, cshape = self.config.as_struct(), shape.as_struct()
-        buffers = BidiBlockSdpaBuffers(view(q), view(local_k), view(local_v), view(q_token_ranges), view(cu_sdpa_partial_outputs),
-                                       view(partial_exp_sums), view(partial_max_logits), view(partial_output))
+        buffers = pack(BidiBlockSdpaBuffers, q, local_k, local_v, q_token_ranges, cu_sdpa_partial_outputs, partial_exp_sums,
+                       partial_max_logits, partial_output)
         _lib.check(_lib.lib().khm_bidi_block_sdpa(ctypes.byref(config), ctypes.byref(cshape), ctypes.byref(buffers), num_active_q_token_ranges,
                                                   param_block(replay_parameters), stream_handle(stream)))

@@ -5,7 +5,7 @@ from __future__ import annotations
 import ctypes
 
 from . import _lib, kv_page_write, rms_norm_rope
-from ._buffers import param_block, stream_handle, view
+from ._buffers import pack, param_block, stream_handle
 from ._lib import KNormRopePageWriteBuffers, ReplayU32
 
 
@@ -21,8 +21,7 @@ class Compute:
     def invoke(self, shape: kv_page_write.Shape, *, pages, k, v, norm_weight, req_slots, flat_token_indices, page_ids,
                num_active_tokens: ReplayU32, page_table_index: ReplayU32, replay_parameters=None, stream=None) -> None:
         norm, page, cshape = self.norm_config.as_struct(), self.page_config.as_struct(), shape.as_struct()
-        buffers = KNormRopePageWriteBuffers(view(pages), view(k), view(v), view(norm_weight), view(req_slots), view(flat_token_indices),
-                                            view(page_ids))
+        buffers = pack(KNormRopePageWriteBuffers, pages, k, v, norm_weight, req_slots, flat_token_indices, page_ids)
         _lib.check(_lib.lib().khm_k_norm_rope_page_write(ctypes.byref(norm), ctypes.byref(page), ctypes.byref(cshape), ctypes.byref(buffers),
                                                          num_active_tokens, page_table_index, param_block(replay_parameters),
                                                          stream_handle(stream)))

@@ -2,10 +2,11 @@
 from __future__ import annotations
 
 import ctypes
+import functools
 from dataclasses import dataclass
 
 from . import _lib
-from ._buffers import param_block, stream_handle, view
+from ._buffers import pack, param_block, stream_handle, view
 from ._lib import DTYPE_BF16, DTYPE_FP8_E4M3FN, KvPageWriteBuffers, KvPageWriteConfig, KvPageWriteShape, PageTableLayoutStruct, ReplayU32
 
 
@@ -35,6 +36,11 @@ class Config:
     dtype: int = DTYPE_BF16
     kv_dtype: int = DTYPE_FP8_E4M3FN
 
+    @functools.cached_property
+    def struct(self) -> KvPageWriteConfig:
+        """`as_struct`, laid out once: the fields are frozen."""
+        return self.as_struct()
+
     def as_struct(self) -> KvPageWriteConfig:
         return KvPageWriteConfig(self.num_kv_heads, self.head_dim, self.page_bytes, self.dtype, self.kv_dtype)
 
@@ -59,6 +65,11 @@ class Shape:
     num_total_token_writes: int
     page_table_layout: PageTableLayout
 
+    @functools.cached_property
+    def struct(self) -> KvPageWriteShape:
+        """`as_struct`, laid out once: the fields are frozen."""
+        return self.as_struct()
+
     def as_struct(self) -> KvPageWriteShape:
         return KvPageWriteShape(self.num_total_token_writes, self.page_table_layout.as_struct())
 
@@ -75,8 +86,8 @@ class Compute:
 
     def invoke(self, shape: Shape, *, pages, flat_k, flat_v, req_slots, flat_token_indices, page_ids, num_active_token_writes: ReplayU32,
                page_table_index: ReplayU32, replay_parameters=None, stream=None) -> None:
-        config, cshape = self.config.as_struct(), shape.as_struct()
-        buffers = KvPageWriteBuffers(view(pages), view(flat_k), view(flat_v), view(req_slots), view(flat_token_indices), view(page_ids))
+        config, cshape = self.config.struct, shape.struct
+        buffers = pack(KvPageWriteBuffers, pages, flat_k, flat_v, req_slots, flat_token_indices, page_ids)
         _lib.check(_lib.lib().khm_kv_page_write(ctypes.byref(config), ctypes.byref(cshape), ctypes.byref(buffers), num_active_token_writes,
                                                 page_table_index, param_block(replay_parameters), stream_handle(stream)))
 

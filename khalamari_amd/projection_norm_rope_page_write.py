@@ -6,8 +6,8 @@ from __future__ import annotations
 import ctypes
 
 from . import _lib, kv_page_write, rms_norm_rope
-from ._buffers import param_block, stream_handle, view
-from ._lib import Buffer, ProjectionNormRopePageWriteBuffers, ReplayU32
+from ._buffers import NO_BUFFER, pack, param_block, stream_handle
+from ._lib import ProjectionNormRopePageWriteBuffers, ReplayU32
 
 
 class Compute:
@@ -29,11 +29,9 @@ class Compute:
     def invoke(self, shape: kv_page_write.Shape, *, projection, q_norm_weight, k_norm_weight, q_output, pages, req_slots, flat_token_indices,
                page_ids, num_active_tokens: ReplayU32, page_table_index: ReplayU32, gate_output=None, replay_parameters=None,
                stream=None) -> None:
-        q_norm, k_norm = self.q_norm_config.as_struct(), self.k_norm_config.as_struct()
-        page, cshape = self.page_config.as_struct(), shape.as_struct()
-        buffers = ProjectionNormRopePageWriteBuffers(view(projection), view(q_norm_weight), view(k_norm_weight), view(q_output),
-                                                     view(gate_output) if gate_output is not None else Buffer(0, 0), view(pages),
-                                                     view(req_slots), view(flat_token_indices), view(page_ids))
+        q_norm, k_norm, page, cshape = self.q_norm_config.struct, self.k_norm_config.struct, self.page_config.struct, shape.struct
+        buffers = pack(ProjectionNormRopePageWriteBuffers, projection, q_norm_weight, k_norm_weight, q_output,
+                       NO_BUFFER if gate_output is None else gate_output, pages, req_slots, flat_token_indices, page_ids)
         _lib.check(_lib.lib().khm_gqa_projection_norm_rope_page_write(
             1 if self.gated else 0, ctypes.byref(q_norm), ctypes.byref(k_norm), ctypes.byref(page), ctypes.byref(cshape), ctypes.byref(buffers),
             num_active_tokens, page_table_index, param_block(replay_parameters), stream_handle(stream)))

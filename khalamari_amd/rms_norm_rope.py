@@ -2,11 +2,12 @@
 from __future__ import annotations
 
 import ctypes
+import functools
 from dataclasses import dataclass, replace
 from typing import Optional
 
 from . import _lib
-from ._buffers import param_block, stream_handle, view
+from ._buffers import pack, param_block, stream_handle
 from ._lib import DTYPE_BF16, DTYPE_F32, ReplayU32, RmsNormRopeBuffers, RmsNormRopeConfig, RopeScalingStruct
 
 
@@ -49,6 +50,11 @@ class Config:
     def with_norm_weight_dtype(self, dtype: int) -> "Config":
         return replace(self, norm_weight_dtype=dtype)
 
+    @functools.cached_property
+    def struct(self) -> RmsNormRopeConfig:
+        """`as_struct`, laid out once: the fields are frozen."""
+        return self.as_struct()
+
     def as_struct(self) -> RmsNormRopeConfig:
         y = self.rope_scaling
         scaling = RopeScalingStruct(0, 1.0, 1.0, 1.0, 1.0, 1, 0) if y is None else RopeScalingStruct(
@@ -86,7 +92,7 @@ class Compute:
 
     def invoke(self, shape: Shape, *, input, norm_weight, flat_token_indices, output, num_active_tokens: ReplayU32, replay_parameters=None,
                stream=None) -> None:
-        config = self.config.as_struct()
-        buffers = RmsNormRopeBuffers(view(input), view(norm_weight), view(flat_token_indices), view(output))
+        config = self.config.struct
+        buffers = pack(RmsNormRopeBuffers, input, norm_weight, flat_token_indices, output)
         _lib.check(_lib.lib().khm_rms_norm_rope(ctypes.byref(config), shape.num_total_tokens, ctypes.byref(buffers), num_active_tokens,
                                                 param_block(replay_parameters), stream_handle(stream)))

@@ -5,7 +5,7 @@ import ctypes
 from dataclasses import dataclass, field
 
 from . import _lib
-from ._buffers import param_block, stream_handle, view
+from ._buffers import NO_BUFFER, pack, param_block, stream_handle, view
 from ._lib import (DTYPE_BF16, GqaSdpaConfig, GqaSdpaShape, PageTableLayout, ReplayU32, SdpaVariant,
                    SlicedKvMapBuffers, SlicedKvReduceBuffers, SlicedKvStaticBuffers)
 
@@ -121,9 +121,8 @@ class Compute:
     def invoke_map(self, *, q, kv_pages, req_slots, page_ids, sdpa_map_task_templates, partial_exp_sums,
                    partial_max_logits, partial_output, page_table_index: ReplayU32, num_active_tokens: ReplayU32,
                    num_active_kv_splits: ReplayU32, replay_parameters=None, stream=None) -> None:
-        buffers = SlicedKvMapBuffers(view(q), view(kv_pages), view(req_slots), view(page_ids),
-                                     view(sdpa_map_task_templates), view(partial_exp_sums), view(partial_max_logits),
-                                     view(partial_output))
+        buffers = pack(SlicedKvMapBuffers, q, kv_pages, req_slots, page_ids, sdpa_map_task_templates, partial_exp_sums, partial_max_logits,
+                       partial_output)
         _lib.check(_lib.lib().khm_sliced_kv_map(self._handle, ctypes.byref(buffers), page_table_index, num_active_tokens,
                                                 num_active_kv_splits, param_block(replay_parameters),
                                                 stream_handle(stream)))
@@ -137,12 +136,10 @@ class Compute:
                           page_table_index: ReplayU32, num_active_tokens: ReplayU32, num_active_kv_splits: ReplayU32,
                           gates=None, replay_parameters=None, stream=None) -> None:
         """Map and Reduce (optionally gated) in one launch; `arrival_counters` must start zeroed."""
-        map_buffers = SlicedKvMapBuffers(view(q), view(kv_pages), view(req_slots), view(page_ids),
-                                         view(sdpa_map_task_templates), view(partial_exp_sums), view(partial_max_logits),
-                                         view(partial_output))
-        reduce_buffers = SlicedKvReduceBuffers(view(partial_exp_sums), view(partial_max_logits), view(partial_output),
-                                               view(cu_sdpa_partial_outputs), view(output))
-        gate_view = view(gates) if gates is not None else _lib.Buffer(None, 0)
+        map_buffers = pack(SlicedKvMapBuffers, q, kv_pages, req_slots, page_ids, sdpa_map_task_templates, partial_exp_sums,
+                           partial_max_logits, partial_output)
+        reduce_buffers = pack(SlicedKvReduceBuffers, partial_exp_sums, partial_max_logits, partial_output, cu_sdpa_partial_outputs, output)
+        gate_view = view(gates) if gates is not None else NO_BUFFER
         _lib.check(_lib.lib().khm_sliced_kv_map_reduce(self._handle, ctypes.byref(map_buffers), ctypes.byref(reduce_buffers),
                                                        gate_view, view(arrival_counters), page_table_index, num_active_tokens,
                                                        num_active_kv_splits, param_block(replay_parameters),
@@ -153,17 +150,15 @@ class Compute:
                                  num_active_kv_splits: ReplayU32, gates=None, replay_parameters=None, stream=None) -> None:
         """`invoke_map_reduce` with the partial states and arrival counters in the library's own static device array:
         nothing is allocated and no workspace is passed (no counterpart in the reference)."""
-        buffers = SlicedKvStaticBuffers(view(q), view(kv_pages), view(req_slots), view(page_ids), view(sdpa_map_task_templates),
-                                        view(cu_sdpa_partial_outputs), view(output))
-        gate_view = view(gates) if gates is not None else _lib.Buffer(None, 0)
+        buffers = pack(SlicedKvStaticBuffers, q, kv_pages, req_slots, page_ids, sdpa_map_task_templates, cu_sdpa_partial_outputs, output)
+        gate_view = view(gates) if gates is not None else NO_BUFFER
         _lib.check(_lib.lib().khm_sliced_kv_map_reduce_static(self._handle, ctypes.byref(buffers), gate_view, page_table_index,
                                                               num_active_tokens, num_active_kv_splits,
                                                               param_block(replay_parameters), stream_handle(stream)))
 
     def invoke_reduce(self, *, partial_exp_sums, partial_max_logits, partial_output, cu_sdpa_partial_outputs, output,
                       num_active_tokens: ReplayU32, gates=None, replay_parameters=None, stream=None) -> None:
-        buffers = SlicedKvReduceBuffers(view(partial_exp_sums), view(partial_max_logits), view(partial_output),
-                                        view(cu_sdpa_partial_outputs), view(output))
+        buffers = pack(SlicedKvReduceBuffers, partial_exp_sums, partial_max_logits, partial_output, cu_sdpa_partial_outputs, output)
         if gates is None:
             _lib.check(_lib.lib().khm_sliced_kv_reduce(self._handle, ctypes.byref(buffers), num_active_tokens,
                                                        param_block(replay_parameters), stream_handle(stream)))

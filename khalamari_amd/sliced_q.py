@@ -5,7 +5,7 @@ import ctypes
 from dataclasses import dataclass
 
 from . import _lib
-from ._buffers import param_block, stream_handle, view
+from ._buffers import pack, param_block, stream_handle, view
 from ._lib import (GqaSdpaShape, ReplayU32, SdpaVariant, SlicedQDirectBuffers, SlicedQMapBuffers, SlicedQReduceBuffers)
 from .sliced_kv import Config as _BaseConfig
 from .sliced_kv import Layout  # noqa: F401
@@ -68,9 +68,8 @@ class Compute:
                    sdpa_map_task_templates, partial_output, partial_exp_sums, partial_max_logits,
                    page_table_index: ReplayU32, num_active_tokens: ReplayU32, num_active_q_token_tiles: ReplayU32,
                    num_active_kv_splits: ReplayU32, replay_parameters=None, stream=None) -> None:
-        buffers = SlicedQMapBuffers(view(q), view(kv_pages), view(req_slots), view(page_ids),
-                                    view(visible_kv_token_ranges), view(q_token_ranges), view(sdpa_map_task_templates),
-                                    view(partial_output), view(partial_exp_sums), view(partial_max_logits))
+        buffers = pack(SlicedQMapBuffers, q, kv_pages, req_slots, page_ids, visible_kv_token_ranges, q_token_ranges, sdpa_map_task_templates,
+                       partial_output, partial_exp_sums, partial_max_logits)
         _lib.check(_lib.lib().khm_sliced_q_map(self._handle, ctypes.byref(buffers), page_table_index, num_active_tokens,
                                                num_active_q_token_tiles, num_active_kv_splits,
                                                param_block(replay_parameters), stream_handle(stream)))
@@ -85,11 +84,10 @@ class Compute:
                           num_active_tokens: ReplayU32, num_active_q_token_tiles: ReplayU32, num_active_kv_splits: ReplayU32,
                           replay_parameters=None, stream=None) -> None:
         """Map and Reduce in one launch; `arrival_counters` must start zeroed."""
-        map_buffers = SlicedQMapBuffers(view(q), view(kv_pages), view(req_slots), view(page_ids),
-                                        view(visible_kv_token_ranges), view(q_token_ranges), view(sdpa_map_task_templates),
-                                        view(partial_output), view(partial_exp_sums), view(partial_max_logits))
-        reduce_buffers = SlicedQReduceBuffers(view(partial_output), view(partial_exp_sums), view(partial_max_logits),
-                                              view(q_token_ranges), view(cu_sdpa_partial_outputs), view(output))
+        map_buffers = pack(SlicedQMapBuffers, q, kv_pages, req_slots, page_ids, visible_kv_token_ranges, q_token_ranges,
+                           sdpa_map_task_templates, partial_output, partial_exp_sums, partial_max_logits)
+        reduce_buffers = pack(SlicedQReduceBuffers, partial_output, partial_exp_sums, partial_max_logits, q_token_ranges,
+                              cu_sdpa_partial_outputs, output)
         _lib.check(_lib.lib().khm_sliced_q_map_reduce(self._handle, ctypes.byref(map_buffers), ctypes.byref(reduce_buffers),
                                                       view(arrival_counters), page_table_index, num_active_tokens,
                                                       num_active_q_token_tiles, num_active_kv_splits,
@@ -99,9 +97,8 @@ class Compute:
                       sdpa_map_task_templates, output, page_table_index: ReplayU32, num_active_tokens: ReplayU32,
                       num_active_q_token_tiles: ReplayU32, replay_parameters=None, stream=None, gates=None) -> None:
         """`gates` (bf16 [T][Hq][D]) fuses the sigmoid gate that follows the SDPA into the output write."""
-        buffers = SlicedQDirectBuffers(view(q), view(kv_pages), view(req_slots), view(page_ids),
-                                       view(visible_kv_token_ranges), view(q_token_ranges),
-                                       view(sdpa_map_task_templates), view(output))
+        buffers = pack(SlicedQDirectBuffers, q, kv_pages, req_slots, page_ids, visible_kv_token_ranges, q_token_ranges,
+                       sdpa_map_task_templates, output)
         if gates is not None:
             _lib.check(_lib.lib().khm_sliced_q_direct_gated(self._handle, ctypes.byref(buffers), view(gates), page_table_index,
                                                             num_active_tokens, num_active_q_token_tiles,
@@ -114,8 +111,7 @@ class Compute:
     def invoke_reduce(self, *, partial_output, partial_exp_sums, partial_max_logits, q_token_ranges,
                       cu_sdpa_partial_outputs, output, num_active_q_token_tiles: ReplayU32, replay_parameters=None,
                       stream=None, gates=None) -> None:
-        buffers = SlicedQReduceBuffers(view(partial_output), view(partial_exp_sums), view(partial_max_logits),
-                                       view(q_token_ranges), view(cu_sdpa_partial_outputs), view(output))
+        buffers = pack(SlicedQReduceBuffers, partial_output, partial_exp_sums, partial_max_logits, q_token_ranges, cu_sdpa_partial_outputs, output)
         if gates is not None:
             _lib.check(_lib.lib().khm_sliced_q_reduce_gated(self._handle, ctypes.byref(buffers), view(gates), num_active_q_token_tiles,
                                                             param_block(replay_parameters), stream_handle(stream)))

@@ -1,0 +1,35 @@
+"""`pack` lays out what one `view` per field would, for everything a buffer can be given as."""
+import pytest
+import torch
+
+from khalamari_amd._buffers import NO_BUFFER, pack, view
+from khalamari_amd._lib import Buffer, RmsNormRopeBuffers, SlicedKvMapBuffers
+
+
+class Borrowed:
+    def data_ptr(self):
+        return 4096
+
+    def numel(self):
+        return 6
+
+    def element_size(self):
+        return 2
+
+
+def test_packed_fields_equal_the_views():
+    tensor = torch.zeros(3, 5, dtype=torch.bfloat16)
+    objects = (tensor, tensor[1:], torch.zeros(0, dtype=torch.int32), (1 << 47, 1 << 40), Buffer(64, 16), NO_BUFFER, Borrowed(), torch.nn.Parameter(torch.ones(7)))
+    packed = pack(SlicedKvMapBuffers, *objects)
+    for (name, _), obj in zip(SlicedKvMapBuffers._fields_, objects):
+        expected, actual = view(obj), getattr(packed, name)
+        assert (actual.ptr, actual.len_bytes) == (expected.ptr, expected.len_bytes), name
+
+
+def test_what_is_no_buffer_is_refused():
+    with pytest.raises(TypeError, match="cannot borrow"):
+        pack(RmsNormRopeBuffers, (1, 2), 7, (1, 2), (1, 2))
+    with pytest.raises(TypeError, match="cannot borrow"):
+        pack(RmsNormRopeBuffers, (1, 2), None, (1, 2), (1, 2))
+    with pytest.raises(ValueError):
+        pack(RmsNormRopeBuffers, (1, 2), (1, 2))   # a field is missing
