@@ -16,8 +16,8 @@
 // passing through registers; NSTAGES tiles are in flight and one barrier per tile publishes them.  A direct load
 // writes 64 consecutive 16-byte chunks, so rows cannot be padded; instead each lane fetches the chunk whose index is
 // XOR-swizzled with the row, which makes both the b128 K reads and the transposed V reads bank-conflict free.
-// Blocks are renumbered so that each XCD walks a contiguous run of the (KV head, active template) list: the Q ranges of
-// one sequence share their K/V through that XCD's L2 instead of each pulling it from HBM.
+// Blocks take head groups fastest and templates last to first (sliced_q_work_item): the Q ranges of one sequence share their
+// K/V through an XCD's L2 instead of each pulling it from HBM.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
