@@ -36,6 +36,8 @@ def pack(struct_type, *objects):
                 add(obj.nbytes)
             except AttributeError:
                 add(obj.numel() * obj.element_size())
+    if len(objects) != len(struct_type._fields_):   # `from_buffer` takes an array that is too long, and later fields would shift
+        raise TypeError(f"{struct_type.__name__} takes {len(struct_type._fields_)} buffers, not {len(objects)}")
     return struct_type.from_buffer(array("Q", words))
 
 

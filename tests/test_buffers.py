@@ -31,5 +31,11 @@ def test_what_is_no_buffer_is_refused():
         pack(RmsNormRopeBuffers, (1, 2), 7, (1, 2), (1, 2))
     with pytest.raises(TypeError, match="cannot borrow"):
         pack(RmsNormRopeBuffers, (1, 2), None, (1, 2), (1, 2))
-    with pytest.raises(ValueError):
+    with pytest.raises((TypeError, ValueError)):
         pack(RmsNormRopeBuffers, (1, 2), (1, 2))   # a field is missing
+
+
+def test_a_surplus_buffer_is_refused():
+    # one more object would shift every field behind it: the kernel would get pointers of other buffers
+    with pytest.raises(TypeError, match="takes 4 buffers, not 5"):
+        pack(RmsNormRopeBuffers, (1, 2), (1, 2), (1, 2), (1, 2), (1, 2))
