@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "block_order.h"
 #include "device_params.h"
 
 namespace khm {
@@ -68,23 +69,9 @@ __device__ __forceinline__ uint32_t active_kv_splits(const MapParams& p) {
     return active;
 }
 
-// Block -> (head group, template) of a sliced-Q launch over `active` templates: head groups fastest, templates last to first.
-// Hardware deals consecutive block ids round-robin to the 8 XCDs, so with 8 KV heads every XCD keeps one head and with 4 or
-// 2 two or four XCDs take turns with a head's templates: the Q ranges of one sequence share their K/V through an XCD's L2, and
-// every XCD gets long and short templates alike.  (A head-major list cut into 8 contiguous runs gave a head's long half
-// to one XCD and its short half to another: whole layer of one prompt of 4150 / 8300 tokens at Hq24/Hkv4/D256 318 / 1126 us,
-// now 265 / 880 us; two of 4200 at Hq16/Hkv2/D256 512 -> 373 us; 8 KV heads the same either way.)  Last to first:
-// within a request the later Q ranges see more keys, so the long blocks start early and the short ones fill the end of the
-// launch.  The padding of a replayed grid comes last.
-struct WorkItem {
-    uint32_t head_group, task;
-    bool live;
-};
-__device__ __forceinline__ WorkItem sliced_q_work_item(uint32_t active) {
-    if (active > gridDim.x) active = gridDim.x;   // a replayed count beyond the shape reads no template behind the table
-    const uint32_t linear = blockIdx.y * gridDim.x + blockIdx.x;
-    const uint32_t rank = linear / gridDim.y;
-    return WorkItem{linear - rank * gridDim.y, active - 1 - rank, rank < active};
+// This block's work item; a replayed count beyond the shape reads no template behind the table.
+__device__ __forceinline__ WorkItem sliced_q_work_item(uint32_t active, uint32_t head_groups) {
+    return sliced_q_work_item(blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x, active, head_groups);
 }
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }

@@ -14,7 +14,7 @@ POISON = 0x4228
 
 
 @pytest.mark.parametrize("hq,hkv,d,fp8", [(8, 1, 128, False), (16, 2, 128, True), (12, 3, 128, False), (24, 4, 256, True), (40, 8, 128, False),
-                                           (36, 9, 128, True)])
+                                           (36, 9, 128, True), (64, 16, 128, False), (60, 20, 128, True), (32, 16, 256, False)])
 @pytest.mark.parametrize("direct", [False, True])
 def test_fixed_and_replayed_counts_give_the_same_bytes(device, hq, hkv, d, fp8, direct):
     import torch
