@@ -42,4 +42,25 @@ constexpr WorkItem sliced_q_work_item(uint32_t x, uint32_t y, uint32_t z, uint32
     return WorkItem{z < full_slices ? within * full_slices + z : full_slices * kNumXcds + within, active - 1 - rank, rank < active};
 }
 
+// The same for tiles that are the only readers of their K/V bytes (verify and drafting blocks): nothing to share, so each XCD takes a run
+// of the head-major list.  Head groups fastest costs these 1 % on average at 2 and 4 KV heads (29 batches of 2..8 tokens a
+// request; 24 requests on 1000..20000 tokens at Hq64/Hkv4/D128 133 -> 141 us, 25 drafting requests at Hq24/Hkv4/D256 on bf16 pages
+// 142 -> 147 us); 8 KV heads are the same list.  Only where the runs are whole head groups or equal parts of one: with 7 or 9 groups
+// they end inside a head (3 requests on 9000..60000 tokens at Hq36/Hkv9/D256 on FP8 pages 99 against 104 us in runs).
+constexpr bool runs_fit_head_groups(uint32_t head_groups) {
+    return head_groups % kNumXcds == 0 || (head_groups < kNumXcds && (head_groups & (head_groups - 1)) == 0);
+}
+
+constexpr WorkItem sole_reader_work_item(uint32_t x, uint32_t y, uint32_t z, uint32_t width, uint32_t height, uint32_t active, uint32_t head_groups) {
+    if (!runs_fit_head_groups(head_groups)) return sliced_q_work_item(x, y, z, width, active, head_groups);
+    if (active > width) active = width;
+    const uint32_t items = active * head_groups;
+    const uint32_t block = (z * height + y) * width + x;   // the grid has no blocks beyond width * head_groups
+    if (block >= items) return WorkItem{0u, 0u, false};
+    const uint32_t run = items / kNumXcds;
+    const uint32_t item = block < run * kNumXcds ? (block % kNumXcds) * run + block / kNumXcds : block;
+    const uint32_t head_group = item / active;
+    return WorkItem{head_group, active - 1 - (item - head_group * active), true};
+}
+
 }  // namespace khm

@@ -702,7 +702,7 @@ static int launch_sliced_q_map(const khm_sliced_q* compute, const khm_buffer& q,
     const uint32_t head_groups = config.num_kv_heads * compute->num_q_head_ranges;
     if (splits == 0) return KHM_OK;
     KHM_REQUIRE((uint64_t)splits * head_groups <= 0xffffffffull, "GQA SplitKV SlicedQ map grid exceeds the u32 block domain");
-    // the split-KV kernel numbers its blocks over the whole grid, the tile kernel over slices of eight head groups
+    // the split-KV kernel numbers its blocks over the whole grid, the tile kernels as block_order.h says
     const dim3 grid = compute->map_merges_in_kernel ? dim3(splits, head_groups, 1)
                                                     : dim3(splits, head_groups_per_slice(head_groups), head_group_slices(head_groups));
     KHM_LAUNCH(compute->map, grid, dim3(compute->map_threads), compute->map_smem_bytes, static_cast<hipStream_t>(stream), p);

@@ -70,8 +70,10 @@ __device__ __forceinline__ uint32_t active_kv_splits(const MapParams& p) {
 }
 
 // This block's work item; a replayed count beyond the shape reads no template behind the table.
-__device__ __forceinline__ WorkItem sliced_q_work_item(uint32_t active, uint32_t head_groups) {
-    return sliced_q_work_item(blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x, active, head_groups);
+template <bool SOLE_READER>
+__device__ __forceinline__ WorkItem work_item_of_block(uint32_t active, uint32_t head_groups) {
+    if constexpr (SOLE_READER) return sole_reader_work_item(blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x, gridDim.y, active, head_groups);
+    else return sliced_q_work_item(blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x, active, head_groups);
 }
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }

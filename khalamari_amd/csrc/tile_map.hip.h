@@ -16,7 +16,7 @@
 // passing through registers; NSTAGES tiles are in flight and one barrier per tile publishes them.  A direct load
 // writes 64 consecutive 16-byte chunks, so rows cannot be padded; instead each lane fetches the chunk whose index is
 // XOR-swizzled with the row, which makes both the b128 K reads and the transposed V reads bank-conflict free.
-// Blocks take head groups fastest and templates last to first (sliced_q_work_item): the Q ranges of one sequence share their
+// Blocks take head groups fastest and templates last to first (block_order.h): the Q ranges of one sequence share their
 // K/V through an XCD's L2 instead of each pulling it from HBM.
 #pragma once
 #include <hip/hip_runtime.h>
@@ -196,7 +196,7 @@ void tile_map_kernel(const MapParams p) {
     // every link of the chain arguments (-> replayed count) -> template -> Q range -> request slot is a scalar load, and what
     // hangs on the same link is requested together (see split_kv_map_kernel)
     fetch_all_arguments(p);
-    const WorkItem item = sliced_q_work_item(active_kv_splits(p), p.num_kv_heads * p.num_q_head_ranges);
+    const WorkItem item = work_item_of_block<STREAM_KV>(active_kv_splits(p), p.num_kv_heads * p.num_q_head_ranges);
     if (!item.live) return;
     const ReplayValues replay = resolve_replay_values(p);
     const uint32_t head_group = item.head_group, task = item.task;
