@@ -128,6 +128,12 @@ __device__ __forceinline__ uint4 load_streaming(const void* source) {
     const U32x4 v = __builtin_nontemporal_load(reinterpret_cast<const U32x4*>(source));
     return make_uint4(v[0], v[1], v[2], v[3]);
 }
+// Sixteen bytes of K/V, kept in the caches or not.
+template <bool SOLE_READER>
+__device__ __forceinline__ uint4 load_kv(const void* source) {
+    if constexpr (SOLE_READER) return load_streaming(source);
+    else return *reinterpret_cast<const uint4*>(source);
+}
 
 __device__ __forceinline__ float bf16_bits_to_f32(uint32_t bits) { return __uint_as_float(bits << 16); }
 

@@ -76,8 +76,9 @@ struct MapTask {
 };
 
 // One block's work.  `smem` holds split_kv_map_smem_bytes.  ACC_IN_AGPRS: the accumulator is held in the AGPR half of the
-// register file (see the end of compute_tile); CAN_MERGE: the call may ask for the Reduce in the last block.
-template <int D, int NT, int NWAVES, bool KV8, bool ACC_IN_AGPRS, bool CAN_MERGE>
+// register file (see the end of compute_tile); CAN_MERGE: the call may ask for the Reduce in the last block; SOLE_READER: no
+// other block of the launch reads these K/V bytes.
+template <int D, int NT, int NWAVES, bool KV8, bool ACC_IN_AGPRS, bool CAN_MERGE, bool SOLE_READER = true>
 __device__ __forceinline__ void split_kv_map_block(const MapParams& p, const MapTask& t, unsigned char* smem) {
     constexpr int KS = D / 32;
     constexpr int MT = D / 16;
@@ -255,7 +256,7 @@ __device__ __forceinline__ void split_kv_map_block(const MapParams& p, const Map
             const uint64_t page = (row >= 8 ? id1 : id0);
             const unsigned char* base = p.kv_pages + page * p.page_bytes + kv_head_row0_k + (uint64_t)in_page * ROW_BYTES + g * 16;
 #pragma unroll
-            for (int i = 0; i < LOADS; ++i) tile.k[i] = load_streaming(base + i * 64);   // this block is the only reader
+            for (int i = 0; i < LOADS; ++i) tile.k[i] = load_kv<SOLE_READER>(base + i * 64);
         }
         {
             const uint32_t row_in_load = lane / LANES_PER_ROW;
@@ -266,7 +267,7 @@ __device__ __forceinline__ void split_kv_map_block(const MapParams& p, const Map
                 const uint32_t in_page = (first_token + row) & (tpp - 1);
                 const uint64_t page = (row >= 8 ? id1 : id0);
                 const unsigned char* source = p.kv_pages + page * p.page_bytes + kv_head_row0_v + (uint64_t)in_page * ROW_BYTES + chunk_in_row * 16;
-                tile.v[i] = load_streaming(source);
+                tile.v[i] = load_kv<SOLE_READER>(source);
             }
         }
     };

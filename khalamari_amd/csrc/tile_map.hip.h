@@ -219,8 +219,14 @@ void tile_map_kernel(const MapParams p) {
         // layer 236.2 -> 220.0 us; 59 of 1000..16000 tokens beside one chunk of 100 389 -> 225 us; bf16 pages 229.4 -> 222.8 us.
         // Four waves, Hq32/Hkv8: 199.9 -> 179.3 and 436 -> 287 us (2048-token chunks without such ranges 3.776 -> 3.799 ms).
         static_assert(split_kv_map_smem_bytes<D, 1, NWAVES, KV8>() <= Smem::kBytes, "the block's LDS holds the decode kernel's");
+        // The last tokens of a chunk make such a range too.  Its K/V are those of the chunk's other ranges and stay in the caches (33
+        // tokens on 4000..8000 cached ones, 16 requests at Hq64/Hkv8 on bf16 pages, layer: streamed 213 us, kept 196 us); those of a
+        // request of its own stream (nine requests with one chunk of 200 at Hq40/Hkv8: streamed 202 us, kept 210 us).
         if (num_q * p.max_q_heads <= 16) {
-            split_kv_map_block<D, 1, NWAVES, KV8, false, false>(p, MapTask{task, head_group, range_index, kv_begin, kv_end, flat_begin, num_q, req_slot, layer, replay.num_active_kv_splits}, tile_smem);
+            const MapTask map_task{task, head_group, range_index, kv_begin, kv_end, flat_begin, num_q, req_slot, layer, replay.num_active_kv_splits};
+            const bool shares = flat_begin > 0 && load_uniform_u32(p.req_slots, flat_begin - 1) == req_slot;
+            if (shares) split_kv_map_block<D, 1, NWAVES, KV8, false, false, false>(p, map_task, tile_smem);
+            else split_kv_map_block<D, 1, NWAVES, KV8, false, false, true>(p, map_task, tile_smem);
             return;
         }
     }

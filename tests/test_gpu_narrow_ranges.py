@@ -1,5 +1,6 @@
 """Q ranges that fill at most one 16-column tile beside wide ones in the same launch (requests that decode beside a chunk): the waves
-of a block share such a range's tokens.  Ranges on both sides of the line, slices off every boundary, NaN in unused slots."""
+of a block share such a range's tokens.  Requests of their own and the last token of a chunk (its K/V are kept in the caches), ranges
+on both sides of the line, slices off every boundary, NaN in unused slots."""
 import pytest
 
 from khalamari_amd import sdpa
