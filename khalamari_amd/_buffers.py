@@ -26,16 +26,19 @@ def pack(struct_type, *objects):
     words = []
     add = words.append
     for obj in objects:
-        if obj.__class__ is Buffer or not hasattr(obj, "data_ptr"):
+        try:
+            nbytes = obj.nbytes   # a tensor, in most calls
+            plain = nbytes.__class__ is int
+            ptr = obj.data_ptr() if plain else 0
+        except AttributeError:
+            plain = False
+        if plain:
+            add(ptr)
+            add(nbytes)
+        else:
             buffer = view(obj)
             add(buffer.ptr or 0)
             add(buffer.len_bytes)
-        else:
-            add(obj.data_ptr())
-            try:
-                add(obj.nbytes)
-            except AttributeError:
-                add(obj.numel() * obj.element_size())
     if len(objects) != len(struct_type._fields_):   # `from_buffer` takes an array that is too long, and later fields would shift
         raise TypeError(f"{struct_type.__name__} takes {len(struct_type._fields_)} buffers, not {len(objects)}")
     return struct_type.from_buffer(array("Q", words))

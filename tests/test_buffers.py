@@ -31,6 +31,8 @@ def test_what_is_no_buffer_is_refused():
         pack(RmsNormRopeBuffers, (1, 2), 7, (1, 2), (1, 2))
     with pytest.raises(TypeError, match="cannot borrow"):
         pack(RmsNormRopeBuffers, (1, 2), None, (1, 2), (1, 2))
+    with pytest.raises(TypeError, match="cannot borrow"):
+        pack(RmsNormRopeBuffers, (1, 2), memoryview(b"host"), (1, 2), (1, 2))   # counts its bytes, but has no device pointer
     with pytest.raises((TypeError, ValueError)):
         pack(RmsNormRopeBuffers, (1, 2), (1, 2))   # a field is missing
 
@@ -39,3 +41,20 @@ def test_a_surplus_buffer_is_refused():
     # one more object would shift every field behind it: the kernel would get pointers of other buffers
     with pytest.raises(TypeError, match="takes 4 buffers, not 5"):
         pack(RmsNormRopeBuffers, (1, 2), (1, 2), (1, 2), (1, 2), (1, 2))
+
+
+class CountsItsBytes(Borrowed):
+    def nbytes(self):
+        return self.numel() * self.element_size()
+
+
+class BorrowedPair(tuple):
+    def data_ptr(self):
+        raise AssertionError("a (pointer, bytes) pair is taken as it is")
+
+
+def test_objects_that_only_view_understands():
+    packed = pack(RmsNormRopeBuffers, CountsItsBytes(), BorrowedPair((64, 16)), (-1, 16), (1, 2))
+    for (name, _), expected in zip(RmsNormRopeBuffers._fields_, (view(CountsItsBytes()), view(BorrowedPair((64, 16))), view((-1, 16)), view((1, 2)))):
+        actual = getattr(packed, name)
+        assert (actual.ptr, actual.len_bytes) == (expected.ptr, expected.len_bytes), name
