@@ -49,8 +49,9 @@ def stream_handle(stream) -> int:
     if stream is None:
         import torch
 
-        # the handle itself; current_stream() builds a Python object around it first
-        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+        # the handle itself, where this torch has it; current_stream() builds a Python object around it first
+        raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+        return int(torch.cuda.current_stream().cuda_stream) if raw is None else raw(torch.cuda.current_device())
     if hasattr(stream, "cuda_stream"):
         return int(stream.cuda_stream)
     return int(stream)

@@ -2,7 +2,7 @@
 import pytest
 import torch
 
-from khalamari_amd._buffers import NO_BUFFER, pack, view
+from khalamari_amd._buffers import NO_BUFFER, pack, stream_handle, view
 from khalamari_amd._lib import Buffer, RmsNormRopeBuffers, SlicedKvMapBuffers
 
 
@@ -58,3 +58,16 @@ def test_objects_that_only_view_understands():
     for (name, _), expected in zip(RmsNormRopeBuffers._fields_, (view(CountsItsBytes()), view(BorrowedPair((64, 16))), view((-1, 16)), view((1, 2)))):
         actual = getattr(packed, name)
         assert (actual.ptr, actual.len_bytes) == (expected.ptr, expected.len_bytes), name
+
+
+class Stream:
+    cuda_stream = 77
+
+
+def test_current_stream_without_the_raw_handle(monkeypatch):
+    # the raw handle is no public name of torch: without it the stream object is asked
+    monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream", raising=False)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: Stream())
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    assert stream_handle(None) == 77
+    assert stream_handle(Stream()) == 77 and stream_handle(5) == 5
