@@ -77,7 +77,7 @@ __device__ __forceinline__ WorkItem work_item_of_block(uint32_t active, uint32_t
 }
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
-// e^x through v_exp_f32; both Reduce implementations use this one so they agree bit for bit.
+// e^x through v_exp_f32, in the Reduce kernels and the Map's last block.
 __device__ __forceinline__ float fast_exp(float x) { return __builtin_amdgcn_exp2f(x * 1.4426950408889634f); }
 
 // Combining one value per 16-lane row over the four rows of a wave (lanes l, l^16, l^32, l^48), result in every lane.

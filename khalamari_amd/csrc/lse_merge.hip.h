@@ -3,7 +3,8 @@
 // Contract of the reference's reducers (gqa_sdpa_sliced_kv_reduce.metal:30-55, gqa_sdpa_sliced_q_reduce.metal:27-62):
 //     w_p = exp(max_p - gmax) * sum_p, 0 for an empty partial;  out = sum_p w_p * partial_p / sum_p w_p.
 // Here the walk over partials is a single online pass (running max, rescale on increase) so that the loads of
-// eight partials can be in flight at once instead of one dependent load per step.
+// several partials can be in flight at once instead of one dependent load per step: eight per lane group in the Map's last
+// block, two to sixteen in the Reduce kernels.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -48,25 +49,15 @@ __device__ __forceinline__ f32x4 bf16x4_to_f32x4(uint32_t a, uint32_t b) {
     return f32x4{bf16_bits_to_f32(a & 0xffffu), bf16_bits_to_f32(a >> 16), bf16_bits_to_f32(b & 0xffffu), bf16_bits_to_f32(b >> 16)};
 }
 
-template <bool COHERENT>
-__device__ __forceinline__ float merge_load_f32(const float* address) {
-    if constexpr (COHERENT) return coherent_load_f32(address);
-    return *address;
-}
-
-template <bool COHERENT>
-__device__ __forceinline__ uint64_t merge_load_u64(const void* address) {
-    if constexpr (COHERENT) return coherent_load_u64(address);
-    return *reinterpret_cast<const uint64_t*>(address);
-}
-
 // Merges partials first, first + step, ... < end of one (Q head, token offset) row into `state`, for the four
-// dims chunk*4 .. chunk*4+3.  `safe_part` is any valid partial index (address of masked-off batch slots).
-template <int D, bool COHERENT, int BATCH = 8>
+// dims chunk*4 .. chunk*4+3.  `safe_part` is any valid partial index (address of masked-off batch slots).  For the Map's
+// last block: other blocks of the same launch wrote the partials, so the loads are device-coherent.
+template <int D>
 __device__ __forceinline__ void merge_partial_slice(MergeState& state, const float* max_logits, const float* exp_sums, const void* partial,
                                                     bool f32_partials, uint32_t first, uint32_t end, uint32_t step, uint32_t safe_part,
                                                     uint32_t num_q_heads, uint32_t q_head, uint32_t max_q_tokens, uint32_t token_offset,
                                                     int chunk) {
+    constexpr int BATCH = 8;
     for (; first < end; first += BATCH * step) {
         float part_max[BATCH], part_sum[BATCH];
         uint64_t lo[BATCH], hi[BATCH];
@@ -75,14 +66,14 @@ __device__ __forceinline__ void merge_partial_slice(MergeState& state, const flo
             const uint32_t part = first + k * step;
             const bool ok = part < end;
             const uint64_t row = ((uint64_t)(ok ? part : safe_part) * num_q_heads + q_head) * max_q_tokens + token_offset;
-            part_max[k] = merge_load_f32<COHERENT>(max_logits + row);
-            part_sum[k] = ok ? merge_load_f32<COHERENT>(exp_sums + row) : 0.0f;
+            part_max[k] = coherent_load_f32(max_logits + row);
+            part_sum[k] = ok ? coherent_load_f32(exp_sums + row) : 0.0f;
             if (f32_partials) {
                 const float* source = reinterpret_cast<const float*>(partial) + row * D + chunk * 4;
-                lo[k] = merge_load_u64<COHERENT>(source);
-                hi[k] = merge_load_u64<COHERENT>(source + 2);
+                lo[k] = coherent_load_u64(source);
+                hi[k] = coherent_load_u64(source + 2);
             } else {
-                lo[k] = merge_load_u64<COHERENT>(reinterpret_cast<const uint16_t*>(partial) + row * D + chunk * 4);
+                lo[k] = coherent_load_u64(reinterpret_cast<const uint16_t*>(partial) + row * D + chunk * 4);
                 hi[k] = 0;
             }
         }

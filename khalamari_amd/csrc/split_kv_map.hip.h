@@ -94,11 +94,13 @@ __device__ __forceinline__ void split_kv_map_block(const MapParams& p, const Map
     // 236 registers instead of 296, so a compute unit holds two blocks (two waves per SIMD) instead of one; these blocks
     // run at the pace of their own load -> decode -> MFMA chain, which a second wave on the SIMD overlaps (four requests of
     // 131072 tokens: 200 -> 194 us).  bf16 pages at D 256 stay at one block either way (399 registers) and are within 3 %
-    // of a read-only launch; at D 128 a third block per CU was measured and changes nothing.
+    // of a read-only launch; at D 128 on bf16 pages a third block per CU was measured and changes nothing.
     // D 128 on FP8 pages: with Q in LDS and the accumulator in ordinary registers (128 of them, 36 AGPRs beside them before) a
     // compute unit holds four blocks instead of three, which a grid of 1024 equal blocks fills in one round instead of one and
     // a third: 45 requests of 300..12000 tokens at Hq64/Hkv8 layer 119.4 -> 112.2 us, 60 of 511..8000 at Hq32/Hkv8 123.8 ->
-    // 115.1 us; four of 131072 in 2048 blocks 194.6 -> 196.0 us.
+    // 115.1 us, 16 of 8192 in 2048 blocks of 512 tokens 63.8 -> 59.5 us.  Many long blocks gain nothing: four requests of 131072 in
+    // 2048 blocks of 2048 tokens 181.1 -> 181.5 us, eight of 100000 in 3136 280.7 -> 282.1 us; the host does not know the
+    // lengths (its count of blocks is the same in both kinds), so they go the same way.
     constexpr bool kSlim = D == 256 && KV8;
     constexpr bool kFourBlocks = D == 128 && KV8;
     constexpr bool kQInRegs = (NT == 1) && !kSlim && !kFourBlocks;
@@ -422,9 +424,10 @@ __device__ __forceinline__ void split_kv_map_block(const MapParams& p, const Map
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
-        // (Not with four blocks per CU, where the wave has 128 registers in all.)
         // The accumulator stays in the AGPR half of the register file from tile to tile (only the rare rescale moves
         // it through VGPRs); without the pin the compiler keeps a second copy in VGPRs and refreshes it after every tile.
+        // Not where the wave has no AGPRs to give: the FP8 build at D 128 (four blocks per CU, 128 registers in all) and
+        // the narrow ranges of a tile kernel, whose wide path takes them as VGPRs.
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
@@ -627,7 +630,7 @@ __device__ __forceinline__ void split_kv_map_block(const MapParams& p, const Map
                 const uint32_t q_head = first_q_head + (live ? local_head : 0u);
                 MergeState state = merge_state_empty();
                 if (live) {
-                    merge_partial_slice<D, true>(state, p.max_logits, p.exp_sums, p.out, f32_partials, partial_begin + slice, partial_end, slices,
+                    merge_partial_slice<D>(state, p.max_logits, p.exp_sums, p.out, f32_partials, partial_begin + slice, partial_end, slices,
                                                  partial_begin, p.num_q_heads, q_head, p.max_q_tokens, token_offset, chunk);
                 }
                 if (slices > 1u) {
@@ -663,7 +666,8 @@ __global__ __launch_bounds__(NWAVES * 64, (KV8 && D == 128) ? 4 : 1) void split_
     // the life of a 512-token decode block: arguments -> task template -> request slot -> page ids -> K/V.  Every link is
     // a scalar load, and everything that hangs on the same link is requested together: the whole argument block; then
     // the template's three words and the replay values; then (sliced-Q) the Q range; then the request slot.  The grid
-    // has one block per template of the padded shape, so reading the template before the activity test is in bounds.
+    // has at most one block per template of the shape and head group (a fixed count: the active ones), so reading the
+    // template before the activity test is in bounds.
     fetch_all_arguments(p);
     const ReplayValues replay = resolve_replay_values(p);
     const uint32_t range_index = load_uniform_u32(p.templates, 3 * (uint64_t)task);

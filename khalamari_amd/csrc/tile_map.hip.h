@@ -134,9 +134,10 @@ void tile_map_kernel(const MapParams p) {
     // id and scalar base.  Otherwise (twelve waves over sixteen units) the 2 * UNITS loads of a tile are dealt out as one
     // list, two or three to a wave, and a wave with fewer repeats its last one so that every wave counts the same number
     // of loads per tile (the waits are compile-time constants).
-    // FP8 tiles staged through registers have half as many units; when there are fewer than waves (twelve waves over
-    // eight units) the first UNITS waves load one unit each and the others none (those loads are ordinary ones the
-    // compiler waits for, so nothing has to be counted).
+    // FP8 tiles have half as many units; when there are fewer than waves (twelve waves over eight units) the first UNITS waves
+    // load one unit each of K and V and the others none.  Staged through registers these are ordinary loads the compiler
+    // waits for; raw codes go straight to LDS, and each loading wave counts its LPW loads per tile like any other, while
+    // the waits of the others return at once and the barrier tells them that the tile is there.
     constexpr int LOADERS = (KV8 && UNITS < NWAVES) ? UNITS : NWAVES;          // waves that load
     constexpr bool PAIRED = UNITS % LOADERS == 0;
     constexpr int UPW = PAIRED ? UNITS / LOADERS : 1;                          // units per loading wave (paired form)
