@@ -13,14 +13,16 @@ pytestmark = pytest.mark.gpu
 POISON = 0x4228
 
 
-@pytest.mark.parametrize("hq,hkv,d,fp8", [(8, 1, 128, False), (16, 2, 128, True), (12, 3, 128, False), (24, 4, 256, True), (40, 8, 128, False),
-                                           (36, 9, 128, True), (64, 16, 128, False), (60, 20, 128, True), (32, 16, 256, False)])
+@pytest.mark.parametrize("hq,hkv,d,fp8,tile", [(8, 1, 128, False, 8), (16, 2, 128, True, 8), (12, 3, 128, False, 8), (24, 4, 256, True, 8),
+                                                (40, 8, 128, False, 8), (36, 9, 128, True, 8), (64, 16, 128, False, 8), (60, 20, 128, True, 8),
+                                                (32, 16, 256, False, 8), (64, 8, 128, False, 32), (64, 8, 128, True, 32), (36, 9, 128, True, 32),
+                                                (12, 3, 256, True, 32), (24, 4, 256, True, 32)])
 @pytest.mark.parametrize("direct", [False, True])
-def test_fixed_and_replayed_counts_give_the_same_bytes(device, hq, hkv, d, fp8, direct):
+def test_fixed_and_replayed_counts_give_the_same_bytes(device, hq, hkv, d, fp8, tile, direct):
     import torch
 
     histories, q_lens = [5, 700, 0, 130, 64], [40, 3, 17, 1, 33]
-    tile, heads = 8, hq // hkv
+    heads = hq // hkv
     w = helpers.make_workload(num_q_heads=hq, num_kv_heads=hkv, head_dim=d, tokens_per_page=16, histories=histories, q_lens=q_lens, seed=hq + d,
                               fp8_pages=fp8)
     ranges, templates, cu = helpers.fixed_slice_plan(histories, q_lens, tile, 4096 if direct else 200)
@@ -63,7 +65,7 @@ def test_fixed_and_replayed_counts_give_the_same_bytes(device, hq, hkv, d, fp8, 
         tokens = int(sum(q_lens[:active_requests]))
         tiles = int(sum(-(-n // tile) for n in q_lens[:active_requests]))
         splits = int(cu[tiles])
-        print(f"padded launch Hq{hq}/Hkv{hkv}/D{d} fp8={fp8} direct={direct} requests={active_requests}", flush=True)
+        print(f"padded launch Hq{hq}/Hkv{hkv}/D{d} fp8={fp8} tile={tile} direct={direct} requests={active_requests}", flush=True)
         params = torch.tensor([tokens, tiles, splits, 0], dtype=torch.int32, device=device)
         fixed = run(*(ReplayU32.fixed(x) for x in (tokens, tiles, splits)), None)
         replayed = run(*(ReplayU32.parameter(i) for i in range(3)), params)

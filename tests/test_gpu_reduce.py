@@ -74,3 +74,39 @@ def test_reduce_against_the_merge_in_float64(device, hq, hkv, d, tile, counts, p
     sigmoid = 1.0 / (1.0 + np.exp(-gates.to(torch.float64).numpy()))
     actual_gated = gated.view(torch.bfloat16).to(torch.float64).cpu().numpy()
     assert np.all(np.abs(actual_gated - actual * sigmoid) <= np.abs(actual) * (4.0 + sigmoid) * 2.0 ** -8)
+
+
+@pytest.mark.parametrize("partial_dtype", [DTYPE_BF16, DTYPE_F32])
+@pytest.mark.parametrize("hq,hkv,d,tile,partials", [(12, 2, 256, 8, 3), (12, 2, 256, 8, 9), (40, 8, 128, 2, 16), (12, 2, 128, 2, 40), (6, 1, 256, 1, 70)])
+def test_reduce_of_buffers_aligned_to_four_bytes(device, hq, hkv, d, tile, partials, partial_dtype):
+    """Every buffer a view that starts four bytes behind a 256-byte boundary: the same bytes as from whole allocations."""
+    import torch
+
+    units, dtype = 5, torch.bfloat16 if partial_dtype == DTYPE_BF16 else torch.float32
+    tokens, templates = units * tile, units * partials
+    generator = torch.Generator(device=device)
+    generator.manual_seed(d + partials)
+    randn = lambda n: torch.randn(n, device=device, generator=generator)  # noqa: E731
+    rows = templates * hq * tile
+    buffers = dict(partial_output=randn(rows * d).to(dtype), partial_exp_sums=randn(rows).abs() + 0.5, partial_max_logits=3.0 * randn(rows),
+                   q_token_ranges=torch.tensor([(i * tile, (i + 1) * tile) for i in range(units)], dtype=torch.int32, device=device).flatten(),
+                   cu_sdpa_partial_outputs=torch.arange(units + 1, dtype=torch.int32, device=device) * partials, gates=randn(tokens * hq * d).to(torch.bfloat16))
+    config = sliced_q.Config(hq, hkv, d, d ** -0.5, 2 * 2 * hkv * 16 * d, sliced_q.Layout(1, 1, 4, 1), partial_dtype=partial_dtype)
+    variant = sdpa.ExecutionVariant.sliced_q(config.sdpa_config(), sdpa.MAP_Q_TOKENS_AND_HEADS, tile, 64, hq // hkv)
+    compute = sliced_q.Compute(config, variant, sliced_q.Shape(tokens, units, templates))
+
+    def shifted(whole):
+        lead = 4 // whole.element_size()
+        view = torch.empty(whole.numel() + lead, dtype=whole.dtype, device=device)[lead:]
+        assert view.data_ptr() % 8 == 4
+        return view.copy_(whole)
+
+    def run(place):
+        output = place(torch.zeros(tokens * hq * d, dtype=torch.bfloat16, device=device))
+        compute.invoke_reduce(output=output, num_active_q_token_tiles=ReplayU32.fixed(units), **{name: place(whole) for name, whole in buffers.items()})
+        torch.cuda.synchronize()
+        return output
+
+    print(f"reduce of shifted buffers Hq{hq} D{d} tile={tile} partials={partials} f32={partial_dtype == DTYPE_F32}", flush=True)
+    whole = run(lambda buffer: buffer)
+    assert bool(whole.any()) and torch.equal(run(shifted).view(torch.int16), whole.view(torch.int16))
