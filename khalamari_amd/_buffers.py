@@ -26,19 +26,18 @@ def pack(struct_type, *objects):
     words = []
     add = words.append
     for obj in objects:
-        try:
-            nbytes = obj.nbytes   # a tensor, in most calls
-            plain = nbytes.__class__ is int
-            ptr = obj.data_ptr() if plain else 0
-        except AttributeError:
-            plain = False
-        if plain:
-            add(ptr)
-            add(nbytes)
-        else:
-            buffer = view(obj)
-            add(buffer.ptr or 0)
-            add(buffer.len_bytes)
+        if obj.__class__ is not Buffer and obj.__class__ is not tuple:
+            try:
+                nbytes = obj.nbytes   # a tensor, in most calls
+                if nbytes.__class__ is int:
+                    add(obj.data_ptr())
+                    add(nbytes)
+                    continue
+            except AttributeError:
+                pass
+        buffer = view(obj)
+        add(buffer.ptr or 0)
+        add(buffer.len_bytes)
     if len(objects) != len(struct_type._fields_):   # `from_buffer` takes an array that is too long, and later fields would shift
         raise TypeError(f"{struct_type.__name__} takes {len(struct_type._fields_)} buffers, not {len(objects)}")
     return struct_type.from_buffer(array("Q", words))
