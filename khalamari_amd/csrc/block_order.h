@@ -42,11 +42,13 @@ constexpr WorkItem sliced_q_work_item(uint32_t x, uint32_t y, uint32_t z, uint32
     return WorkItem{z < full_slices ? within * full_slices + z : full_slices * kNumXcds + within, active - 1 - rank, rank < active};
 }
 
-// The same for tiles that are the only readers of their K/V bytes (verify and drafting blocks): nothing to share, so each XCD takes a run
-// of the head-major list.  Head groups fastest costs these 1 % on average at 2 and 4 KV heads (29 batches of 2..8 tokens a
-// request; 24 requests on 1000..20000 tokens at Hq64/Hkv4/D128 133 -> 141 us, 25 drafting requests at Hq24/Hkv4/D256 on bf16 pages
-// 142 -> 147 us); 8 KV heads are the same list.  Only where the runs are whole head groups or equal parts of one: with 7 or 9 groups
-// they end inside a head (3 requests on 9000..60000 tokens at Hq36/Hkv9/D256 on FP8 pages 99 against 104 us in runs).
+// The same for tiles of bf16 pages that are the only readers of their K/V bytes (verify and drafting blocks): nothing to share, so each
+// XCD takes a run of the head-major list.  On caches that no pass has read before, against head groups fastest: 25 drafting
+// requests on 1200..12000 tokens at Hq24/Hkv4/D256 148.2 -> 143.6 us, 30 verify requests on 1200..24000 at Hq16/Hkv2/D256
+// 180.9 -> 178.1 us, 24 on 1000..20000 at Hq64/Hkv4/D128 139 -> 130 us, 15 on 1200..5000 at Hq32/Hkv4 44.4 -> 44.8 us; 33 such
+// batches 0.8 % faster on average.  FP8 pages are as fast either way (25 batches 0.1 % slower in runs, 33 requests on 400..1500 tokens at
+// Hq24/Hkv4/D256 37.9 -> 40.0 us).  Only where the runs are whole head groups or equal parts of one: with 7 or 9 groups they end
+// inside a head (24 requests at Hq36/Hkv9/D128 223 against 228 us in runs).  8 KV heads are the same list.
 constexpr bool runs_fit_head_groups(uint32_t head_groups) {
     return head_groups % kNumXcds == 0 || (head_groups < kNumXcds && (head_groups & (head_groups - 1)) == 0);
 }

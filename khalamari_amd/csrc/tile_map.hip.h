@@ -197,7 +197,7 @@ void tile_map_kernel(const MapParams p) {
     // every link of the chain arguments (-> replayed count) -> template -> Q range -> request slot is a scalar load, and what
     // hangs on the same link is requested together (see split_kv_map_kernel)
     fetch_all_arguments(p);
-    const WorkItem item = work_item_of_block<STREAM_KV>(active_kv_splits(p), p.num_kv_heads * p.num_q_head_ranges);
+    const WorkItem item = work_item_of_block<STREAM_KV && !KV8>(active_kv_splits(p), p.num_kv_heads * p.num_q_head_ranges);
     if (!item.live) return;
     const ReplayValues replay = resolve_replay_values(p);
     const uint32_t head_group = item.head_group, task = item.task;
