@@ -2,6 +2,7 @@
 from __future__ import annotations
 
 from array import array
+from ctypes import sizeof
 
 from ._lib import Buffer
 
@@ -25,20 +26,20 @@ def pack(struct_type, *objects):
     projection prologue with its configs 13.5 -> 6.4 us of host time; that step as a whole 25.4 -> 15.6 us)."""
     words = []
     add = words.append
-    for obj in objects:
-        if obj.__class__ is not Buffer and obj.__class__ is not tuple:
-            try:
-                nbytes = obj.nbytes   # a tensor, in most calls
-                if nbytes.__class__ is int:
-                    add(obj.data_ptr())
-                    add(nbytes)
-                    continue
-            except AttributeError:
-                pass
-        buffer = view(obj)
-        add(buffer.ptr or 0)
-        add(buffer.len_bytes)
-    if len(objects) != len(struct_type._fields_):   # `from_buffer` takes an array that is too long, and later fields would shift
+    try:
+        for obj in objects:
+            nbytes = getattr(obj, "nbytes", None)
+            if nbytes.__class__ is int:   # a tensor
+                add(obj.data_ptr())
+                add(nbytes)
+            else:
+                buffer = view(obj)
+                add(buffer.ptr or 0)
+                add(buffer.len_bytes)
+    except AttributeError:
+        view(obj)   # says what cannot be borrowed
+        raise
+    if 8 * len(words) != sizeof(struct_type):   # `from_buffer` takes an array that is too long, and later fields would shift
         raise TypeError(f"{struct_type.__name__} takes {len(struct_type._fields_)} buffers, not {len(objects)}")
     return struct_type.from_buffer(array("Q", words))
 
@@ -48,9 +49,11 @@ def stream_handle(stream) -> int:
     if stream is None:
         import torch
 
-        # the handle itself, where this torch has it; current_stream() builds a Python object around it first
-        raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
-        return int(torch.cuda.current_stream().cuda_stream) if raw is None else raw(torch.cuda.current_device())
+        try:
+            # the handle itself; current_stream() builds a Python object around it first
+            return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+        except AttributeError:   # no public name of torch
+            return int(torch.cuda.current_stream().cuda_stream)
     if hasattr(stream, "cuda_stream"):
         return int(stream.cuda_stream)
     return int(stream)
