@@ -34,12 +34,16 @@ constexpr uint32_t head_group_slices(uint32_t head_groups) { return (head_groups
 
 constexpr WorkItem sliced_q_work_item(uint32_t x, uint32_t y, uint32_t z, uint32_t total, uint32_t active, uint32_t head_groups) {
     const uint32_t full_slices = head_groups / kNumXcds;
-    const uint32_t groups = z < full_slices ? kNumXcds : head_groups % kNumXcds;
     const uint32_t linear = y * total + x;
-    const uint32_t rank = linear / groups;
-    const uint32_t within = linear - rank * groups;
+    uint32_t rank = linear / kNumXcds;
+    uint32_t head_group = linear % kNumXcds * full_slices + z;
+    if (z >= full_slices) {
+        const uint32_t groups = head_groups % kNumXcds;
+        rank = linear / groups;
+        head_group = full_slices * kNumXcds + linear - rank * groups;
+    }
     if (active > total) active = total;
-    return WorkItem{z < full_slices ? within * full_slices + z : full_slices * kNumXcds + within, active - 1 - rank, rank < active};
+    return WorkItem{head_group, active - 1 - rank, rank < active};
 }
 
 // The same for tiles of bf16 pages that are the only readers of their K/V bytes (verify and drafting blocks): nothing to share, so each
