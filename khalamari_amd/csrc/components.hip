@@ -241,6 +241,7 @@ static void fill_map_geometry(const ComputeBase& c, MapParams* p) {
     p->num_kv_heads = config.num_kv_heads;
     p->q_heads_per_kv_head = config.num_q_heads / config.num_kv_heads;
     p->max_q_heads = c.variant.map_max_q_heads;
+    p->max_q_heads_reciprocal = 65536 / c.variant.map_max_q_heads + 1;
     p->num_q_head_ranges = c.num_q_head_ranges;
     p->max_q_tokens = c.variant.map_max_q_tokens;
     p->tokens_per_page = c.tokens_per_page;

@@ -38,6 +38,7 @@ struct MapParams {
     uint32_t num_kv_heads;
     uint32_t q_heads_per_kv_head;
     uint32_t max_q_heads;                // Q heads per block (<= q_heads_per_kv_head)
+    uint32_t max_q_heads_reciprocal;     // 65536 / max_q_heads + 1: (c * it) >> 16 is c / max_q_heads for the columns c < 256 of a block
     uint32_t num_q_head_ranges;          // ceil(q_heads_per_kv_head / max_q_heads)
     uint32_t max_q_tokens;               // Q tokens per range (1 for sliced-KV)
     uint32_t tokens_per_page;            // 8, 16 or 32

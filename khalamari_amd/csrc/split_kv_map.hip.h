@@ -135,7 +135,7 @@ __device__ __forceinline__ void split_kv_map_block(const MapParams& p, const Map
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
         const uint32_t c = nt * 16 + r16;
-        const uint32_t token_offset = c / p.max_q_heads;
+        const uint32_t token_offset = token_of_column(p, c);
         const uint32_t local_head = c - token_offset * p.max_q_heads;
         col_active[nt] = token_offset < num_q && local_head < num_heads;
         uint32_t lo = kv_begin, hi = kv_end;
@@ -158,13 +158,11 @@ __device__ __forceinline__ void split_kv_map_block(const MapParams& p, const Map
             all_hi = hi < all_hi ? hi : all_hi;
         }
     }
-#pragma unroll
-    for (int offset = 1; offset < 16; offset <<= 1) {
-        uint32_t other;
-        other = __shfl_xor(blk_lo, offset); blk_lo = other < blk_lo ? other : blk_lo;
-        other = __shfl_xor(blk_hi, offset); blk_hi = other > blk_hi ? other : blk_hi;
-        other = __shfl_xor(all_lo, offset); all_lo = other > all_lo ? other : all_lo;
-        other = __shfl_xor(all_hi, offset); all_hi = other < all_hi ? other : all_hi;
+    if (p.visible_ranges != nullptr) {   // without visible ranges every column sees the template's
+        blk_lo = min_within_row(blk_lo);
+        blk_hi = max_within_row(blk_hi);
+        all_lo = max_within_row(all_lo);
+        all_hi = min_within_row(all_hi);
     }
     blk_lo = __builtin_amdgcn_readfirstlane(blk_lo);
     blk_hi = __builtin_amdgcn_readfirstlane(blk_hi);
@@ -181,7 +179,7 @@ __device__ __forceinline__ void split_kv_map_block(const MapParams& p, const Map
     uint4 q_frag[kQInRegs ? KS : 1];
     if constexpr (kQInRegs) {
         const uint32_t c = r16;
-        const uint32_t token_offset = c / p.max_q_heads;
+        const uint32_t token_offset = token_of_column(p, c);
         const uint32_t local_head = c - token_offset * p.max_q_heads;
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) q_frag[ks] = make_uint4(0, 0, 0, 0);
@@ -195,7 +193,7 @@ __device__ __forceinline__ void split_kv_map_block(const MapParams& p, const Map
         for (int index = tid; index < COLS * Q_CHUNKS; index += NWAVES * 64) {
             const uint32_t c = index / Q_CHUNKS;
             const uint32_t chunk = index - c * Q_CHUNKS;
-            const uint32_t token_offset = c / p.max_q_heads;
+            const uint32_t token_offset = token_of_column(p, c);
             const uint32_t local_head = c - token_offset * p.max_q_heads;
             uint4 value = make_uint4(0, 0, 0, 0);
             if (token_offset < num_q && local_head < num_heads) {
@@ -529,7 +527,7 @@ __device__ __forceinline__ void split_kv_map_block(const MapParams& p, const Map
     for (int index = tid; index < COLS * (D / 4); index += NWAVES * 64) {
         const uint32_t c = index / (D / 4);
         const uint32_t d = (index - c * (D / 4)) * 4;
-        const uint32_t token_offset = c / p.max_q_heads;
+        const uint32_t token_offset = token_of_column(p, c);
         const uint32_t local_head = c - token_offset * p.max_q_heads;
         if (token_offset >= num_q || local_head >= num_heads) continue;
         f32x4 value = *reinterpret_cast<const f32x4*>(o_lds + c * Smem::kORowFloats + d);
@@ -565,7 +563,7 @@ __device__ __forceinline__ void split_kv_map_block(const MapParams& p, const Map
     }
     if (mode != kMapDirectBf16 && tid < COLS) {
         const uint32_t c = tid;
-        const uint32_t token_offset = c / p.max_q_heads;
+        const uint32_t token_offset = token_of_column(p, c);
         const uint32_t local_head = c - token_offset * p.max_q_heads;
         if (token_offset < num_q && local_head < num_heads) {
             const uint64_t state = ((uint64_t)task * p.num_q_heads + first_q_head + local_head) * p.max_q_tokens + token_offset;
@@ -624,7 +622,7 @@ __device__ __forceinline__ void split_kv_map_block(const MapParams& p, const Map
                 const bool has_unit = unit < num_units;
                 const uint32_t c = has_unit ? unit / slices : 0u;
                 const uint32_t slice = unit - c * slices;
-                const uint32_t token_offset = c / p.max_q_heads;
+                const uint32_t token_offset = token_of_column(p, c);
                 const uint32_t local_head = c - token_offset * p.max_q_heads;
                 const bool live = has_unit && local_head < num_heads;
                 const uint32_t q_head = first_q_head + (live ? local_head : 0u);

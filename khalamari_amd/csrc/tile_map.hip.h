@@ -240,15 +240,15 @@ void tile_map_kernel(const MapParams p) {
     const uint32_t first_q_head = kv_head * p.q_heads_per_kv_head + head_range_begin;
 
     // ---- per-lane column facts ---------------------------------------------------------------------------
-    auto column_token = [&](int nt) { return (uint32_t)((wave * NTW + nt) * 16 + r16) / p.max_q_heads; };
-    auto column_head = [&](int nt) { return (uint32_t)((wave * NTW + nt) * 16 + r16) % p.max_q_heads; };
+    auto column_token = [&](int nt) { return token_of_column(p, (wave * NTW + nt) * 16 + r16); };
+    auto column_head = [&](int nt) { return (wave * NTW + nt) * 16 + r16 - column_token(nt) * p.max_q_heads; };
     uint32_t col_lo[NTW], col_hi[NTW];
     bool col_active[NTW];
     uint32_t blk_lo = 0xffffffffu, blk_hi = 0u, wave_all_lo = 0u, wave_all_hi = 0xffffffffu, min_span = 0xffffffffu;
 #pragma unroll
     for (int nt = 0; nt < NTW; ++nt) {
         const uint32_t c = (wave * NTW + nt) * 16 + r16;
-        const uint32_t token_offset = c / p.max_q_heads;
+        const uint32_t token_offset = token_of_column(p, c);
         const uint32_t local_head = c - token_offset * p.max_q_heads;
         col_active[nt] = token_offset < num_q && local_head < num_heads;
         uint32_t lo = kv_begin, hi = kv_end;
@@ -273,15 +273,11 @@ void tile_map_kernel(const MapParams p) {
             min_span = hi - lo < min_span ? hi - lo : min_span;
         }
     }
-#pragma unroll
-    for (int offset = 1; offset < 16; offset <<= 1) {
-        uint32_t other;
-        other = __shfl_xor(blk_lo, offset); blk_lo = other < blk_lo ? other : blk_lo;
-        other = __shfl_xor(blk_hi, offset); blk_hi = other > blk_hi ? other : blk_hi;
-        other = __shfl_xor(wave_all_lo, offset); wave_all_lo = other > wave_all_lo ? other : wave_all_lo;
-        other = __shfl_xor(wave_all_hi, offset); wave_all_hi = other < wave_all_hi ? other : wave_all_hi;
-        other = __shfl_xor(min_span, offset); min_span = other < min_span ? other : min_span;
-    }
+    blk_lo = min_within_row(blk_lo);
+    blk_hi = max_within_row(blk_hi);
+    wave_all_lo = max_within_row(wave_all_lo);
+    wave_all_hi = min_within_row(wave_all_hi);
+    min_span = min_within_row(min_span);
     // A wave none of whose columns is active (a request with fewer Q tokens than the tile has slots, fewer Q heads than
     // the tile has columns for) still loads its share of every K/V tile and meets every barrier, but computes nothing:
     // its LDS reads and matrix instructions would only take issue slots from the waves it shares a SIMD with.
