@@ -138,6 +138,12 @@ void tile_map_kernel(const MapParams p) {
     static_assert((SL == 1 || SL == 2) && NSTAGES >= 3 && NSTAGES <= 5, "unsupported tiling");
     constexpr bool RAW8 = KV8 && NTW == 1;       // raw FP8 codes in LDS, decoded by the waves that read them
     constexpr bool STAGED8 = KV8 && !RAW8;       // FP8 tiles decoded once on their way into bf16 LDS tiles
+    // The steady-state loop for hi + lo weights: 23 verify requests at Hq24/Hkv4/D256 on FP8 pages, layer 116.4 -> 108.1 us, on bf16 pages
+    // 12 of 300..8000 tokens 78.6 -> 74.3; nine prompts of 20..900 tokens at Hq24/Hkv4/D256 147 -> 142 us, at Hq16/Hkv2 109 -> 102, at Hq64/Hkv8/D128
+    // 169 -> 166; 20 drafting requests at Hq32 on bf16 pages 123 -> 118.  Nothing to give where the tile is decoded in registers
+    // (prompts at Hq64 on FP8 pages 171.6 -> 171.5 us, mixed batches 216.7 -> 219.0), and the twelve waves with partial states lose
+    // (mixed batch at Hq24/Hkv4/D256 107 -> 110 us).
+    constexpr bool PRECISE_STEADY = !STAGED8 && (NWAVES < 12 || DIRECT);
     static_assert(!STAGED8 || NSTAGES == 4, "the register-staged FP8 path is written for a ring of four tiles");
     using Smem = TileSmem<D, BK, NSTAGES, RAW8 ? D : 2 * D, LINEAR>;
     constexpr int ROW = Smem::kRowBytes;
@@ -811,7 +817,7 @@ void tile_map_kernel(const MapParams p) {
     // [tile_begin, tile_end) has its successor's first slice in the range, and the tile NSTAGES - 1 ahead exists and lies
     // wholly inside the block's KV range.  One straight-line body per tile: a fixed wait, the barrier, unconditional
     // requests; the compiler is free to mix the S^T of the next slice with the softmax of this one.
-    auto run_steady_tiles = [&](auto untracked_anchored, uint32_t tile_begin, uint32_t tile_end) __attribute__((always_inline)) {
+    auto run_steady_tiles = [&](auto precise_tag, auto untracked_anchored, uint32_t tile_begin, uint32_t tile_end) __attribute__((always_inline)) {
         constexpr std::false_type no{};
         TileIds ahead = fetch_ids_interior(tile_begin + NSTAGES - 1);
         // The loop's place in the lines of the instruction cache does not depend on the length of the task decode in front of it: the
@@ -838,10 +844,10 @@ void tile_map_kernel(const MapParams p) {
             auto nothing = []() __attribute__((always_inline)) {};
             const unsigned char* k_following = k_lds + next_stage * Smem::kKTileBytes;
             if constexpr (SL == 2) {
-                process_slice(no, no, untracked_anchored, 0u, pending, k_tile, k_tile + kKSliceBytes, v_tile, request_next);
-                process_slice(no, no, untracked_anchored, 0u, pending, k_tile + kKSliceBytes, k_following, v_tile + kVSliceBytes, nothing);
+                process_slice(precise_tag, no, untracked_anchored, 0u, pending, k_tile, k_tile + kKSliceBytes, v_tile, request_next);
+                process_slice(precise_tag, no, untracked_anchored, 0u, pending, k_tile + kKSliceBytes, k_following, v_tile + kVSliceBytes, nothing);
             } else {
-                process_slice(no, no, untracked_anchored, 0u, pending, k_tile, k_following, v_tile, request_next);
+                process_slice(precise_tag, no, untracked_anchored, 0u, pending, k_tile, k_following, v_tile, request_next);
             }
         }
     };
@@ -898,21 +904,29 @@ void tile_map_kernel(const MapParams p) {
         tail_begin = tail_begin > head_end ? tail_begin : head_end;
         constexpr std::true_type yes{};
         constexpr std::false_type no{};
+        // tiles t with t + NSTAGES - 1 a whole tile inside [blk_lo, blk_hi), (t + NSTAGES) * BK <= blk_hi - first_token, run in
+        // the steady-state loop
+        uint32_t steady_limit = head_end;
+        {
+            const uint32_t whole_tiles = (blk_hi - first_token) / BK;
+            steady_limit = whole_tiles >= (uint32_t)NSTAGES ? whole_tiles - (NSTAGES - 1) : 0;
+            steady_limit = steady_limit < tail_begin ? steady_limit : tail_begin;
+            steady_limit = steady_limit > head_end ? steady_limit : head_end;
+        }
         if (precise) {
             run_tiles(yes, yes, no, 0, head_end);
-            run_tiles(yes, no, no, head_end, tail_begin);
+            uint32_t general_begin = head_end;
+            if constexpr (PRECISE_STEADY) {
+                if (steady_limit > head_end) {
+                    run_steady_tiles(yes, no, head_end, steady_limit);
+                    upcoming = fetch_ids(steady_limit + NSTAGES - 1);
+                    general_begin = steady_limit;
+                }
+            }
+            run_tiles(yes, no, no, general_begin, tail_begin);
             run_tiles(yes, yes, no, tail_begin, num_tiles);
         } else {
             run_tiles(no, yes, no, 0, head_end);
-            // tiles t with t + NSTAGES - 1 a whole tile inside [blk_lo, blk_hi), (t + NSTAGES) * BK <= blk_hi - first_token, run in
-            // the steady-state loop
-            uint32_t steady_limit = head_end;
-            {
-                const uint32_t whole_tiles = (blk_hi - first_token) / BK;
-                steady_limit = whole_tiles >= (uint32_t)NSTAGES ? whole_tiles - (NSTAGES - 1) : 0;
-                steady_limit = steady_limit < tail_begin ? steady_limit : tail_begin;
-                steady_limit = steady_limit > head_end ? steady_limit : head_end;
-            }
             if constexpr (DIRECT) {
                 // no partial state to hand on: the interior slices need not follow the largest score
 #pragma unroll
@@ -924,14 +938,14 @@ void tile_map_kernel(const MapParams p) {
                     steady_begin = head_end + 1;
                 }
                 if (steady_limit > steady_begin) {
-                    run_steady_tiles(std::integral_constant<int, 2>{}, steady_begin, steady_limit);
+                    run_steady_tiles(no, std::integral_constant<int, 2>{}, steady_begin, steady_limit);
                     upcoming = fetch_ids(steady_limit + NSTAGES - 1);
                     steady_begin = steady_limit;
                 }
                 run_tiles(no, no, yes, steady_begin, tail_begin);
             } else {
                 if (steady_limit > head_end) {
-                    run_steady_tiles(no, head_end, steady_limit);
+                    run_steady_tiles(no, no, head_end, steady_limit);
                     upcoming = fetch_ids(steady_limit + NSTAGES - 1);
                 }
                 run_tiles(no, no, no, steady_limit, tail_begin);
