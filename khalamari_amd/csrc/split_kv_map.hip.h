@@ -68,7 +68,7 @@ constexpr int kMapPrefetchDepth = 2;
 
 // Bytes of LDS a block works in.
 template <int D, int NT, int NWAVES, bool KV8>
-constexpr int split_kv_map_smem_bytes() { return MapSmem<D, NT, NWAVES, NT != 1 || KV8>::kTotal; }
+constexpr int split_kv_map_smem_bytes() { return MapSmem<D, NT, NWAVES, NT != 1 || KV8 || D == 256>::kTotal; }
 
 // What a block knows about its task; everything is block-uniform.
 struct MapTask {
@@ -90,18 +90,21 @@ __device__ __forceinline__ void split_kv_map_block(const MapParams& p, const Map
     constexpr int LOADS = KvTile<D, KV8>::kLoads;
     // first dim of the eight that lane group g contracts in k-step ks (the K fragments above fix the order)
     auto q_dim = [](int ks, int g) { return KV8 ? (ks >> 1) * 64 + g * 16 + (ks & 1) * 8 : ks * 32 + g * 8; };
-    // D 256 on FP8 pages: with the Q fragments read from LDS and one tile requested ahead instead of two the kernel takes
-    // 236 registers instead of 296, so a compute unit holds two blocks (two waves per SIMD) instead of one; these blocks
-    // run at the pace of their own load -> decode -> MFMA chain, which a second wave on the SIMD overlaps (four requests of
-    // 131072 tokens: 200 -> 194 us).  bf16 pages at D 256 stay at one block either way (399 registers) and are within 3 %
-    // of a read-only launch; at D 128 on bf16 pages a third block per CU was measured and changes nothing.
+    // D 256: with the Q fragments read from LDS and one tile requested ahead instead of two a compute unit holds two blocks (two
+    // waves per SIMD) instead of one; these blocks run at the pace of their own load -> product chain, which a second wave on the
+    // SIMD overlaps.  FP8 pages: 236 registers instead of 296, four requests of 131072 tokens 200 -> 194 us.  bf16 pages: 240, which
+    // takes an accumulator in ordinary registers (with it pinned to AGPRs the compiler wanted 396), instead of 396; layers at
+    // Hq24/Hkv4: 12 requests of 200..3000 tokens 39.0 -> 33.4 us, 24 of 200..6000 85.4 -> 77.8, 60 of 200..8000 192 -> 182, one of 3000
+    // 25.7 -> 25.0, four of 60000 in slices of 2048 169 -> 165; 16 at Hq16/Hkv2 54.2 -> 43.7.  (On FP8 pages ordinary registers
+    // take 174 and win and lose 1 to 2 % by batch; two tiles ahead there likewise.)  At D 128 on bf16 pages, 212 registers and
+    // two blocks, a third block loses up to 10 % and a fourth 16 to 40 %.
     // D 128 on FP8 pages: with Q in LDS and the accumulator in ordinary registers (128 of them, 36 AGPRs beside them before) a
     // compute unit holds four blocks instead of three, which a grid of 1024 equal blocks fills in one round instead of one and
     // a third: 45 requests of 300..12000 tokens at Hq64/Hkv8 layer 119.4 -> 112.2 us, 60 of 511..8000 at Hq32/Hkv8 123.8 ->
     // 115.1 us, 16 of 8192 in 2048 blocks of 512 tokens 63.8 -> 59.5 us.  Many long blocks gain nothing: four requests of 131072 in
     // 2048 blocks of 2048 tokens 181.1 -> 181.5 us, eight of 100000 in 3136 280.7 -> 282.1 us; the host does not know the
     // lengths (its count of blocks is the same in both kinds), so they go the same way.
-    constexpr bool kSlim = D == 256 && KV8;
+    constexpr bool kSlim = D == 256;
     constexpr bool kFourBlocks = D == 128 && KV8;
     constexpr bool kQInRegs = (NT == 1) && !kSlim && !kFourBlocks;
     using Smem = MapSmem<D, NT, NWAVES, !kQInRegs>;
@@ -424,8 +427,8 @@ __device__ __forceinline__ void split_kv_map_block(const MapParams& p, const Map
         __builtin_amdgcn_wave_barrier();
         // The accumulator stays in the AGPR half of the register file from tile to tile (only the rare rescale moves
         // it through VGPRs); without the pin the compiler keeps a second copy in VGPRs and refreshes it after every tile.
-        // Not where the wave has no AGPRs to give: the FP8 build at D 128 (four blocks per CU, 128 registers in all) and
-        // the narrow ranges of a tile kernel, whose wide path takes them as VGPRs.
+        // Not where the wave has no AGPRs to give: the FP8 build at D 128 (four blocks per CU, 128 registers in all), the bf16
+        // build at D 256 (two, 240 registers) and the narrow ranges of a tile kernel, whose wide path takes them as VGPRs.
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
@@ -651,7 +654,7 @@ __device__ __forceinline__ void split_kv_map_block(const MapParams& p, const Map
 }
 
 template <int D, int NT, int NWAVES, bool KV8 = false>
-__global__ __launch_bounds__(NWAVES * 64, (KV8 && D == 128) ? 4 : 1) void split_kv_map_kernel(const MapParams p) {
+__global__ __launch_bounds__(NWAVES * 64, KV8 ? (D == 128 ? 4 : 1) : (D == 256 ? 2 : 1)) void split_kv_map_kernel(const MapParams p) {
     __shared__ __align__(16) unsigned char smem[split_kv_map_smem_bytes<D, NT, NWAVES, KV8>()];
     // ---- task decode (uniform) -------------------------------------------------------------
     // Blocks are dispatched in linear order; the KV heads of one task vary fastest, so the blocks in flight together
@@ -688,7 +691,7 @@ __global__ __launch_bounds__(NWAVES * 64, (KV8 && D == 128) ? 4 : 1) void split_
     if (num_q > p.max_q_tokens) num_q = p.max_q_tokens;
     const uint32_t req_slot = load_uniform_u32(p.req_slots, flat_begin);
     const uint32_t layer = replay.layer;
-    split_kv_map_block<D, NT, NWAVES, KV8, !(KV8 && D == 128), true>(p, MapTask{task, head_group_index, range_index, kv_begin, kv_end, flat_begin, num_q, req_slot, layer, num_active_splits}, smem);
+    split_kv_map_block<D, NT, NWAVES, KV8, KV8 == (D == 256), true>(p, MapTask{task, head_group_index, range_index, kv_begin, kv_end, flat_begin, num_q, req_slot, layer, num_active_splits}, smem);
 }
 
 }  // namespace khm
