@@ -161,6 +161,18 @@ def test_gpu_matches_oracle_over_shapes(device, hq, hkv, d, block, max_q, dtype_
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("hq,hkv,d,block,max_q", [
+    (8, 2, 128, 1, 1),       # one key, one token
+    (40, 8, 128, 7, 16),     # ranges that span request blocks, sixteen keys not filled, two blocks of four KV heads
+    (24, 6, 128, 16, 5),     # the sixteen keys filled, a KV head count that leaves waves idle, ranges cut inside a request block
+    (48, 4, 256, 4, 8),      # 96 columns of a KV head: six tiles, every second of a range's request blocks
+    (16, 1, 256, 15, 16),    # one KV head
+])
+def test_gpu_small_blocks_on_the_matrix_cores(device, hq, hkv, d, block, max_q):
+    test_gpu_matches_oracle_over_shapes(device, hq, hkv, d, block, max_q, True)
+
+
+@pytest.mark.gpu
 def test_gpu_replay_active_q_token_ranges(device):
     """test_replay_active_q_token_ranges_match_cpu_reference (bidi_block_sdpa_test.rs:50-157)."""
     import torch
