@@ -176,6 +176,8 @@ extern "C" int khm_gqa_metadata_create(uint64_t max_tokens, uint64_t max_map_tas
         if (status == hipSuccess) status = hipMemset(metadata->device[i], 0, bytes);  // new_zeroed_elements
         block_words += metadata->capacity[i];
     }
+    // the first update may come on a stream that doesn't wait for the null stream
+    if (status == hipSuccess) status = hipStreamSynchronize(nullptr);
     for (StagingBlock& block : metadata->staging) {
         // coherent: the kernel sees what the host wrote before its launch, whatever an earlier launch read from the block
         if (status == hipSuccess) status = hipHostMalloc(reinterpret_cast<void**>(&block.words), block_words * sizeof(uint32_t), hipHostMallocCoherent);
