@@ -32,7 +32,6 @@ NUM_POOLS = 3
 # two `rocprofv3 --pmc` runs per config, each counter scaled by what it reads for a plain 1 GiB copy kernel
 # (`--calibration-copy`).  The summaries with their commands are the text files under profiles/.
 MEASURED_MAP_TRAFFIC_BYTES = {2: 565_561_344, 3: 2_153_930_752, 4: 1_446_890_496, 5: 1_202_827_264, 6: 1_068_915_712}
-# 6 on FP8 pages: the register-staged twelve-wave tile, with its spills; tile_map_fp8_kernel has not been counted.
 MEASURED_MAP_TRAFFIC_BYTES_FP8_PAGES = {2: 286_631_936, 3: 1_082_411_008, 4: 729_135_104, 5: 869_629_952, 6: 1_614_041_088}
 
 CONFIGS = {
@@ -306,14 +305,12 @@ class Workload:
 
     def map_kernel_name(self) -> str:
         """Name of the HIP kernel the Map launch runs: one 16-column tile (decode) uses the split-KV kernel whose waves
-        share nothing, wider Q tiles the LDS-tiled kernel, or the one whose matrix operands are FP8 codes."""
+        share nothing, wider Q tiles the LDS-tiled kernel."""
         coordinates = int(self.variant.map_max_q_tokens) * int(self.variant.map_max_q_heads)
         from khalamari_amd import sdpa
 
         if self.variant.map_kind == sdpa.MAP_SLICED_KV or coordinates <= 16:
             return "split_kv_map_kernel"
-        if self.fp8_pages and 64 < coordinates <= (256 if self.spec["d"] == 256 else 128):
-            return "tile_map_fp8_kernel"
         return "tile_map_kernel"
 
     def step(self, i: int) -> None:

@@ -12,7 +12,6 @@
 #include "reduce_gate.hip.h"
 #include "split_kv_map.hip.h"
 #include "tile_map.hip.h"
-#include "tile_map_fp8.hip.h"
 
 namespace khm {
 
@@ -43,66 +42,62 @@ struct TileKernelChoice {
     uint32_t smem_bytes;
 };
 
-// Prefill tiles on FP8 pages.
-template <int D, int NTW, int NWAVES, int MIN_BLOCKS>
-static TileKernelChoice tile_fp8_choice() {
-    return {tile_map_fp8_kernel<D, NTW, NWAVES, MIN_BLOCKS>, NWAVES * 64, (uint32_t)tile_map_fp8_smem_bytes<D, NWAVES>()};
-}
-
-// FP8 pages.  Which arithmetic a tile has depends on how often its waves would decode the codes.  Verify tiles (four waves, few of
-// them with columns) keep raw codes in LDS and decode what they read.  The 256-column tile at head dim 128 decodes a tile once for
-// eight waves and has bf16 products: splitting the weights into E4M3 pieces costs the vector pipe more than that (2048-token
-// chunks on 0..16384 at Hq64/Hkv8, Map 4.30 ms, with pieces 4.98 ms in one block of eight waves or two of four).  In between,
-// where every conversion serves one or two column tiles or a weight serves 256 dims, the codes are operands as they are:
-// layer of 3 chunks of 130..246 tokens on 35000..40000 at Hq24/Hkv4/D256 735 -> 470 us, 4 of 1000..2048 on up to 8000 there 1000 -> 740 us,
-// at Hq16/Hkv2/D256 (128 columns) 700 -> 550 us, at Hq32/Hkv8/D128 (128 columns) 830 -> 545 us; 24-token prompts of one request at
-// Hq16/Hkv2/D256 16.6 -> 17.3 us (a step is 128 tokens, however few there are).
-static TileKernelChoice select_fp8_tile_kernel(uint32_t head_dim, uint32_t coordinates, bool direct) {
-    if (head_dim == 128) {
-        // BK 64 and a fifth stage were measured slower (170 / 167 us against 165 us on a batch of 16 speculative blocks)
-        if (coordinates <= 64) return {tile_map_kernel<128, 1, 4, 32, 4, 2, true>, 256, (uint32_t)TileSmem<128, 32, 4, 128>::kBytes};
-        if (coordinates <= 128) return tile_fp8_choice<128, 2, 4, 2>();
-        if (direct) return {tile_map_kernel<128, 2, 8, 64, 4, 1, true, true>, 512, (uint32_t)TileSmem<128, 64, 4>::kBytes};
-        return {tile_map_kernel<128, 2, 8, 64, 4, 1, true>, 512, (uint32_t)TileSmem<128, 64, 4>::kBytes};
-    }
-    if (head_dim == 256) {
-        // 64 KB of raw codes per block, so a compute unit has room for two, and a batch of 23 speculative requests on
-        // 1000..20000 tokens (Hq24/Hkv4, 434 MB) needs them: one block (294 registers, one wave per SIMD) leaves every
-        // wait of its tile chain bare, 180 us; two (222 registers) 112 us.
-        if (coordinates <= 64) return {tile_map_kernel<256, 1, 4, 32, 4, 2, true>, 256, (uint32_t)TileSmem<256, 32, 4, 256>::kBytes};
-        if (coordinates <= 128) return tile_fp8_choice<256, 1, 8, 1>();
-        if (coordinates <= 192) return tile_fp8_choice<256, 1, 12, 1>();
-        return tile_fp8_choice<256, 2, 8, 1>();
-    }
-    return {nullptr, 0, 0};
-}
-
 // Tiled (LDS-shared K/V) kernel for Q tiles of 17..256 coordinates: speculative-verify blocks (one 16-column tile per
 // wave, bandwidth-bound) up to prefill tiles (32 columns per wave, MFMA-bound).
 static TileKernelChoice select_tile_kernel(uint32_t head_dim, uint32_t coordinates, uint32_t kv_dtype, bool direct) {
-    if (kv_dtype == KHM_DTYPE_FP8_E4M3FN) return select_fp8_tile_kernel(head_dim, coordinates, direct);
     // The MFMA-bound tiles have a build of their own for computes that only ever write final output: its interior slices
     // do not follow the largest score.  (One kernel holding both kinds of interior loop spills.)  These are the two-
     // column-tile kernels at D 128 and the eight-wave tile at D 256 (523 -> 638 TFLOP/s on 2048-token chunks at
     // Hq24/Hkv4); the bandwidth-bound verify tiles have nothing to gain.
     // Twelve waves of one column tile each for 129..192 coordinates at D 256 (32 tokens x 6 Q heads of a KV head: no idle
-    // column, three waves per SIMD).
+    // column, three waves per SIMD), on bf16 and on FP8 pages.
     if (head_dim == 256 && coordinates > 128 && coordinates <= 192) {
+        if (kv_dtype == KHM_DTYPE_FP8_E4M3FN) {
+            if (direct) return {tile_map_kernel<256, 1, 12, 32, 4, 1, true, true>, 768, (uint32_t)TileSmem<256, 32, 4>::kBytes};
+            return {tile_map_kernel<256, 1, 12, 32, 4, 1, true>, 768, (uint32_t)TileSmem<256, 32, 4, 256>::kBytes};
+        }
         if (direct) return {tile_map_kernel<256, 1, 12, 32, 4, 1, false, true>, 768, (uint32_t)TileSmem<256, 32, 4, 512, true>::kBytes};
         return {tile_map_kernel<256, 1, 12, 32, 4, 1>, 768, (uint32_t)TileSmem<256, 32, 4, 512, true>::kBytes};
     }
-    if (direct && head_dim == 256 && coordinates > 64 && coordinates <= 128)
+    if (direct && head_dim == 256 && coordinates > 64 && coordinates <= 128) {
+        if (kv_dtype == KHM_DTYPE_FP8_E4M3FN)
+            return {tile_map_kernel<256, 1, 8, 32, 4, 1, true, true>, 512, (uint32_t)TileSmem<256, 32, 4>::kBytes};
         return {tile_map_kernel<256, 1, 8, 32, 4, 1, false, true>, 512, (uint32_t)TileSmem<256, 32, 4, 512, true>::kBytes};
+    }
     if (direct && head_dim == 128 && coordinates > 64) {
-        if (coordinates > 128) return {tile_map_kernel<128, 2, 8, 64, 4, 1, false, true>, 512, (uint32_t)TileSmem<128, 64, 4, 256, true>::kBytes};
+        const bool wide = coordinates > 128;
+        if (kv_dtype == KHM_DTYPE_FP8_E4M3FN) {
+            if (wide) return {tile_map_kernel<128, 2, 8, 64, 4, 1, true, true>, 512, (uint32_t)TileSmem<128, 64, 4>::kBytes};
+            return {tile_map_kernel<128, 2, 4, 64, 4, 2, true, true>, 256, (uint32_t)TileSmem<128, 64, 4>::kBytes};
+        }
+        if (wide) return {tile_map_kernel<128, 2, 8, 64, 4, 1, false, true>, 512, (uint32_t)TileSmem<128, 64, 4, 256, true>::kBytes};
         return {tile_map_kernel<128, 1, 8, 32, 4, 2, false, true>, 512, (uint32_t)TileSmem<128, 32, 4, 256, true>::kBytes};
+    }
+    if (kv_dtype == KHM_DTYPE_FP8_E4M3FN) {
+        if (head_dim == 128) {
+            // verify tiles keep the raw codes in LDS (32 KB per block) and decode at the consumer: BK 64 and a fifth stage
+            // were measured slower (170 / 167 us against 165 us on a batch of 16 speculative blocks)
+            if (coordinates <= 64) return {tile_map_kernel<128, 1, 4, 32, 4, 2, true>, 256, (uint32_t)TileSmem<128, 32, 4, 128>::kBytes};   // raw codes in LDS
+            if (coordinates <= 128) return {tile_map_kernel<128, 2, 4, 64, 4, 2, true>, 256, (uint32_t)TileSmem<128, 64, 4>::kBytes};
+            return {tile_map_kernel<128, 2, 8, 64, 4, 1, true>, 512, (uint32_t)TileSmem<128, 64, 4>::kBytes};
+        }
+        if (head_dim == 256) {
+            // Raw codes in LDS: 64 KB per block, so a compute unit has room for two, and a batch of 23 speculative requests on
+            // 1000..20000 tokens (Hq24/Hkv4, 434 MB) needs them: one block (294 registers, one wave per SIMD) leaves every
+            // wait of its tile chain bare, 180 us; two (222 registers) 112 us.
+            if (coordinates <= 64) return {tile_map_kernel<256, 1, 4, 32, 4, 2, true>, 256, (uint32_t)TileSmem<256, 32, 4, 256>::kBytes};
+            if (coordinates <= 128) return {tile_map_kernel<256, 1, 8, 32, 4, 1, true>, 512, (uint32_t)TileSmem<256, 32, 4>::kBytes};
+            return {tile_map_kernel<256, 2, 8, 32, 4, 1, true>, 512, (uint32_t)TileSmem<256, 32, 4>::kBytes};
+        }
+        return {nullptr, 0, 0};
     }
     if (head_dim == 128) {
         if (coordinates <= 64)
             return {tile_map_kernel<128, 1, 4, 32, 4, 2>, 256, (uint32_t)TileSmem<128, 32, 4, 256, true>::kBytes};  // 64 KB: two blocks per CU
         // 65..128 coordinates on bf16 pages: eight waves of one column tile each, BK 32, 64 KB of LDS, two blocks per CU =
         // four waves per SIMD at 118 VGPRs.  A batch of 2048-token chunks held to 128 columns: 5.13 ms, against 6.93 ms
-        // on four waves of two column tiles with BK 64 (and 5.77 ms on eight waves with BK 64 at one block per CU).
+        // on four waves of two column tiles with BK 64 (and 5.77 ms on eight waves with BK 64 at one block per CU).  FP8
+        // pages keep the four-wave tile: a 32-token FP8 tile has fewer load units than eight waves.
         if (coordinates <= 128) return {tile_map_kernel<128, 1, 8, 32, 4, 2>, 512, (uint32_t)TileSmem<128, 32, 4, 256, true>::kBytes};
         return {tile_map_kernel<128, 2, 8, 64, 4, 1>, 512, (uint32_t)TileSmem<128, 64, 4, 256, true>::kBytes};
     }

@@ -80,13 +80,6 @@ __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_ex
 // e^x through v_exp_f32, in the Reduce kernels and the Map's last block.
 __device__ __forceinline__ float fast_exp(float x) { return __builtin_amdgcn_exp2f(x * 1.4426950408889634f); }
 
-// The largest of three, a NaN counting as nothing (fmaxf has a canonicalising instruction in front of each operand).
-__device__ __forceinline__ float max_of_three(float a, float b, float c) {
-    float result;
-    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(result) : "v"(a), "v"(b), "v"(c));
-    return result;
-}
-
 // Combining one value per 16-lane row over the four rows of a wave (lanes l, l^16, l^32, l^48), result in every lane.
 // gfx950 swaps lane rows inside the VALU (v_permlane16_swap / v_permlane32_swap); a generic shuffle would go through
 // the LDS crossbar, whose result also queues behind every LDS read in flight.
@@ -96,12 +89,6 @@ __device__ __forceinline__ float max_over_rows(float x) {
     bits = __float_as_uint(fmaxf(__uint_as_float(halves[0]), __uint_as_float(halves[1])));
     halves = __builtin_amdgcn_permlane32_swap(bits, bits, false, false);
     return fmaxf(__uint_as_float(halves[0]), __uint_as_float(halves[1]));
-}
-__device__ __forceinline__ uint32_t min_over_rows(uint32_t x) {
-    auto halves = __builtin_amdgcn_permlane16_swap(x, x, false, false);
-    x = halves[0] < halves[1] ? halves[0] : halves[1];
-    halves = __builtin_amdgcn_permlane32_swap(x, x, false, false);
-    return halves[0] < halves[1] ? halves[0] : halves[1];
 }
 __device__ __forceinline__ float sum_over_rows(float x) {
     uint32_t bits = __float_as_uint(x);

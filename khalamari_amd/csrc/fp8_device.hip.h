@@ -25,103 +25,6 @@ __device__ __forceinline__ uint4 fp8x8_to_bf16x8(uint2 codes) {
                       fp8x2_to_bf16x2<true>(codes.y));
 }
 
-// ---- FP8 matrix products with a split operand --------------------------------------------------------------------------
-// v_mfma_scale_f32_16x16x128_f8f6f4 takes the page codes as they are, at twice the rate of the bf16 form.  The other operand is a
-// sum of E4M3 pieces, each 2^-4 of the one before: piece n holds value * 2^(4 n), and its product carries the block scale 2^(-4 n).
-typedef int i32x8 __attribute__((ext_vector_type(8)));
-constexpr float kPieceStep = 0x1p-4f;
-constexpr int kPieceScale0 = 0x7f7f7f7f, kPieceScale1 = 0x7b7b7b7b, kPieceScale2 = 0x77777777;   // E8M0: 2^0, 2^-4, 2^-8
-
-// a register whose contents do not matter: the conversions fill one half of theirs at a time, and a zero would be an instruction
-__device__ __forceinline__ int any_bits() {
-    int bits;
-    asm volatile("" : "=v"(bits));   // volatile: one for each use, not one register copied about
-    return bits;
-}
-__device__ __forceinline__ uint32_t f32x4_to_fp8x4(float a, float b, float c, float d) {
-    const int low = __builtin_amdgcn_cvt_pk_fp8_f32(a, b, any_bits(), false);
-    return (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(c, d, low, true);
-}
-// codes of x / scale (scale a power of two)
-__device__ __forceinline__ uint32_t f32x4_to_scaled_fp8x4(float a, float b, float c, float d, float scale) {
-    typedef short S16x2 __attribute__((ext_vector_type(2)));
-    const S16x2 low = __builtin_amdgcn_cvt_scalef32_pk_fp8_f32(__builtin_bit_cast(S16x2, any_bits()), a, b, scale, false);
-    return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_fp8_f32(low, c, d, scale, true));
-}
-// what the codes leave of x (exact: the remainder of a rounding)
-__device__ __forceinline__ void subtract_fp8x4(float (&x)[4], uint32_t codes) {
-    const auto low = __builtin_amdgcn_cvt_pk_f32_fp8((int)codes, false), high = __builtin_amdgcn_cvt_pk_f32_fp8((int)codes, true);
-    x[0] -= low[0];
-    x[1] -= low[1];
-    x[2] -= high[0];
-    x[3] -= high[1];
-}
-__device__ __forceinline__ void subtract_scaled_fp8x4(float (&x)[4], uint32_t codes, float scale) {
-    const auto low = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(codes, scale, false), high = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(codes, scale, true);
-    x[0] -= low[0];
-    x[1] -= low[1];
-    x[2] -= high[0];
-    x[3] -= high[1];
-}
-// c + A . (B * scale): A are page codes, B one piece
-__device__ __forceinline__ f32x4 mfma_fp8_k128(i32x8 a, i32x8 b, f32x4 c, int piece_scale) {
-    return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, c, 0, 0, 0, kPieceScale0, 0, piece_scale);
-}
-
-// A row of bf16 values as two pieces: scaled by a power of two so that the row's largest value lies in [2^7, 2^8), a value is four
-// significant bits and a remainder of at most eight of its own units, both exact from 2^-14 of the largest on.  A row with an
-// infinity keeps the signs of the infinite values, beside which the finite ones are nothing, and has an infinite scale; a NaN
-// stays one.
-struct SplitScale {
-    float unit;      // the power of two a code is worth
-    bool infinite;
-    __device__ __forceinline__ float column_scale() const { return infinite ? INFINITY : unit; }
-};
-struct SplitCodes {
-    uint2 high, low;
-};
-// the two bf16 magnitudes of `largest` and eight more, the larger of each position
-__device__ __forceinline__ uint32_t largest_magnitudes(uint4 bits, uint32_t largest) {
-    typedef unsigned short U16x2 __attribute__((ext_vector_type(2)));
-    const uint32_t words[4] = {bits.x, bits.y, bits.z, bits.w};
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-        largest = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(U16x2, words[i] & 0x7fff7fffu), __builtin_bit_cast(U16x2, largest)));
-    return largest;
-}
-__device__ __forceinline__ uint32_t larger_half(uint32_t pair) { return (pair & 0xffffu) > (pair >> 16) ? (pair & 0xffffu) : (pair >> 16); }
-__device__ __forceinline__ SplitScale split_scale_of(uint32_t largest_magnitude) {
-    uint32_t exponent = largest_magnitude >> 7;
-    exponent = exponent < 16u ? 16u : (exponent > 254u ? 254u : exponent);   // the unit and a sixteenth of it are normal numbers
-    return SplitScale{__uint_as_float((exponent - 7u) << 23), largest_magnitude == 0x7f80u};
-}
-__device__ __forceinline__ SplitCodes split_bf16x8(uint4 bits, const SplitScale& scale) {
-    typedef short S16x2 __attribute__((ext_vector_type(2)));
-    uint32_t words[4] = {bits.x, bits.y, bits.z, bits.w};
-    if (__builtin_amdgcn_ballot_w64(scale.infinite) != 0) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            if (!scale.infinite) continue;
-            // 2^127 = 128 units of such a row (its exponent counts as 254)
-            const uint32_t low = (words[i] & 0x7fffu) == 0x7f80u ? (words[i] & 0x8000u) | 0x7f00u : 0u;
-            const uint32_t high = ((words[i] >> 16) & 0x7fffu) == 0x7f80u ? ((words[i] >> 16) & 0x8000u) | 0x7f00u : 0u;
-            words[i] = low | (high << 16);
-        }
-    }
-    uint32_t high[2], low[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const S16x2 first = __builtin_amdgcn_cvt_scalef32_pk_fp8_bf16(__builtin_bit_cast(S16x2, any_bits()), __builtin_bit_cast(bf16x2, words[2 * i]), scale.unit, false);
-        high[i] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_fp8_bf16(first, __builtin_bit_cast(bf16x2, words[2 * i + 1]), scale.unit, true));
-        float x[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) x[j] = j & 1 ? __uint_as_float(words[2 * i + j / 2] & 0xffff0000u) : bf16_bits_to_f32(words[2 * i + j / 2]);
-        subtract_scaled_fp8x4(x, high[i], scale.unit);
-        low[i] = f32x4_to_scaled_fp8x4(x[0], x[1], x[2], x[3], scale.unit * kPieceStep);
-    }
-    return SplitCodes{make_uint2(high[0], high[1]), make_uint2(low[0], low[1])};
-}
-
 // One bf16 bit pattern to its E4M3FN code, in integer arithmetic on the bf16 fields (7-bit mantissa -> 3 bits).
 __device__ __forceinline__ uint32_t bf16_bits_to_fp8_e4m3fn(uint32_t bits) {
     const uint32_t sign = (bits >> 8) & 0x80u;

@@ -106,7 +106,11 @@ __device__ __forceinline__ void barrier_keeping_loads_in_flight() {
 // is one ds_read_b64, a V^T fragment one ds_read_b64_tr_b8, four conversions each).  That repeats the decode in each of
 // the four waves, which these tiles have the VALU time for, and takes the chain load -> registers -> decode -> LDS ->
 // barrier off the critical path of a tile.
-// (Head dim 256, and up to 128 coordinates at head dim 128, have a kernel of their own above 64 coordinates: tile_map_fp8.hip.h.)
+// The twelve-wave tile at head dim 256 has 168 registers per wave.  With the staged tile in them its partial-state build (which
+// follows the largest score) spilled 86, among them the Q fragments, and every slice waited for them to come back from
+// scratch; with raw codes in LDS it takes 166 and none spills, at half the LDS reads: 511 tokens on 35000..40000 cached ones at
+// Hq24/Hkv4 815 -> 705 us, decode beside two 500-token chunks (layer) 381 -> 282 us.  The direct-output build keeps the staged tile: its
+// interior loop holds its Q fragments, and decoding in all twelve waves costs it more (2048-token chunks 4.02 -> 4.88 ms).
 // DIRECT: the instantiation only ever writes final output (p.output_mode == kMapDirectBf16, which the host guarantees);
 // it exists where following the largest score is worth compiling out, see the untracked slices below.
 template <int D, int NTW, int NWAVES, int BK, int NSTAGES, int MIN_BLOCKS, bool KV8 = false, bool DIRECT = false>
@@ -130,13 +134,20 @@ void tile_map_kernel(const MapParams p) {
     // id and scalar base.  Otherwise (twelve waves over sixteen units) the 2 * UNITS loads of a tile are dealt out as one
     // list, two or three to a wave, and a wave with fewer repeats its last one so that every wave counts the same number
     // of loads per tile (the waits are compile-time constants).
-    constexpr bool PAIRED = UNITS % NWAVES == 0;
-    constexpr int UPW = PAIRED ? UNITS / NWAVES : 1;                          // units per loading wave (paired form)
+    // FP8 tiles have half as many units; when there are fewer than waves (twelve waves over eight units) the first UNITS waves
+    // load one unit each of K and V and the others none.  Staged through registers these are ordinary loads the compiler
+    // waits for; raw codes go straight to LDS, and each loading wave counts its LPW loads per tile like any other, while
+    // the waits of the others return at once and the barrier tells them that the tile is there.
+    constexpr int LOADERS = (KV8 && UNITS < NWAVES) ? UNITS : NWAVES;          // waves that load
+    constexpr bool PAIRED = UNITS % LOADERS == 0;
+    constexpr int UPW = PAIRED ? UNITS / LOADERS : 1;                          // units per loading wave (paired form)
     constexpr int LPW = PAIRED ? 2 * UPW : (2 * UNITS + NWAVES - 1) / NWAVES;  // loads per wave and tile
     constexpr int IDS = PAIRED ? UPW : LPW;                                    // page ids per wave and tile
     static_assert(PAIRED || !KV8, "FP8 tiles are written for evenly divided units");
+    static_assert(LOADERS == NWAVES || KV8, "only FP8 tiles leave waves without loads");
     static_assert((SL == 1 || SL == 2) && NSTAGES >= 3 && NSTAGES <= 5, "unsupported tiling");
-    constexpr bool RAW8 = KV8 && NTW == 1;       // raw FP8 codes in LDS, decoded by the waves that read them
+    // raw FP8 codes in LDS, decoded by the waves that read them (the twelve-wave tile: partial-state build only, see above)
+    constexpr bool RAW8 = KV8 && NTW == 1 && (NWAVES == 4 || (NWAVES == 12 && !DIRECT));
     constexpr bool STAGED8 = KV8 && !RAW8;       // FP8 tiles decoded once on their way into bf16 LDS tiles
     // The steady-state loop for hi + lo weights: 23 verify requests at Hq24/Hkv4/D256 on FP8 pages, layer 116.4 -> 108.1 us, on bf16 pages
     // 12 of 300..8000 tokens 78.6 -> 74.3; nine prompts of 20..900 tokens at Hq24/Hkv4/D256 147 -> 142 us, at Hq16/Hkv2 109 -> 102, at Hq64/Hkv8/D128
@@ -401,7 +412,9 @@ void tile_map_kernel(const MapParams p) {
         lane_offset[j] = ((first_token + source.row) & (tpp - 1)) * PAGE_ROW + (source.chunk << 4) + (load_is_v(j) ? v_plane_distance : 0u);
     }
     const unsigned char* const k_plane_base = p.kv_pages + plane_k;
+    const bool wave_loads = LOADERS == NWAVES || wave < LOADERS;   // wave-uniform; a wave without loads waits for none
     auto issue_tile = [&](uint32_t tile, const TileIds ids) __attribute__((always_inline)) {
+        if (!wave_loads) return;
         const uint32_t stage = tile % NSTAGES;
         const uint32_t tile_token = first_token + tile * BK;
         if (tile_token >= blk_lo && tile_token + BK <= blk_hi) {
@@ -435,6 +448,7 @@ void tile_map_kernel(const MapParams p) {
         return ids;
     };
     auto issue_interior_tile = [&](uint32_t stage, const TileIds ids) __attribute__((always_inline)) {
+        if (!wave_loads) return;
 #pragma unroll
         for (int j = 0; j < LPW; ++j)
             load_to_lds_b128<STREAM_KV>(k_plane_base + (uint64_t)ids[load_id(j)] * p.page_bytes, lane_offset[j], load_lds_address(j, stage));
@@ -444,6 +458,7 @@ void tile_map_kernel(const MapParams p) {
     // (source chunk c of a K row lands at position c ^ (row & 15), of a V row at c ^ 2 (row & 7)).
     uint4 raw_k[STAGED8 ? UPW : 1], raw_v[STAGED8 ? UPW : 1];
     auto load_raw_tile = [&](uint32_t tile, const TileIds ids) __attribute__((always_inline)) {
+        if (!wave_loads) return;
         const uint32_t load_row = lane / CPR;
         const uint32_t load_pos = lane % CPR;
         const uint32_t tile_token = first_token + tile * BK;
@@ -466,6 +481,7 @@ void tile_map_kernel(const MapParams p) {
             raw_lane_offset[i] = ((first_token + (wave * UPW + i) * RPL + lane / CPR) & (tpp - 1)) * PAGE_ROW + (lane % CPR) * 16;
     }
     auto load_raw_tile_interior = [&](const TileIds ids) __attribute__((always_inline)) {
+        if (!wave_loads) return;
 #pragma unroll
         for (int i = 0; i < UPW; ++i) {
             const unsigned char* page = k_plane_base + (uint64_t)ids[i] * p.page_bytes;
@@ -474,6 +490,7 @@ void tile_map_kernel(const MapParams p) {
         }
     };
     auto write_raw_tile = [&](uint32_t tile) __attribute__((always_inline)) {
+        if (!wave_loads) return;
         const uint32_t load_row = lane / CPR;
         const uint32_t load_pos = lane % CPR;
         unsigned char* k_stage = k_lds + (tile % NSTAGES) * Smem::kKTileBytes;

@@ -126,3 +126,23 @@ def run_sliced_q(w, ranges, templates, cu, device, *, kind, max_q_tokens, max_q_
                               num_active_q_token_tiles=ReplayU32.fixed(ranges.shape[0]), gates=gates_d)
     torch.cuda.synchronize()
     return bf16_tensor_to_f32(out)
+
+
+def run_sliced_q_map(w, ranges, templates, device, *, kind, max_q_tokens, max_q_heads, stage=64):
+    """The Map alone with float32 partial states: f32 [templates][Hq][max_q_tokens][D], zeros where no row was written."""
+    g = w.geom
+    config = component_config(w, sliced_q.Config, DTYPE_F32)
+    variant = sdpa.ExecutionVariant.sliced_q(config.sdpa_config(), kind, max_q_tokens, stage, max_q_heads)
+    shape = sliced_q.Shape(w.num_tokens, ranges.shape[0], templates.shape[0])
+    compute = sliced_q.Compute(config, variant, shape, direct=False)
+    partial = torch.zeros(config.partial_output_bytes(variant, shape), dtype=torch.uint8, device=device)
+    sums = torch.zeros(config.partial_output_stats_bytes(variant, shape), dtype=torch.uint8, device=device)
+    maxs = torch.zeros_like(sums)
+    compute.invoke_map(q=to_device(w.q_bits, device), kv_pages=to_device(w.kv_pages, device), req_slots=to_device(w.req_slots, device),
+                       page_ids=to_device(w.page_ids, device), visible_kv_token_ranges=to_device(w.visible, device),
+                       q_token_ranges=to_device(ranges, device), sdpa_map_task_templates=to_device(templates, device), partial_output=partial,
+                       partial_exp_sums=sums, partial_max_logits=maxs, page_table_index=ReplayU32.fixed(w.layer),
+                       num_active_tokens=ReplayU32.fixed(w.num_tokens), num_active_q_token_tiles=ReplayU32.fixed(ranges.shape[0]),
+                       num_active_kv_splits=ReplayU32.fixed(templates.shape[0]))
+    torch.cuda.synchronize()
+    return partial.view(torch.float32).reshape(templates.shape[0], g.num_q_heads, max_q_tokens, g.head_dim).cpu().numpy()
