@@ -246,8 +246,16 @@ void tile_map_kernel(const MapParams p) {
     const uint32_t first_q_head = kv_head * p.q_heads_per_kv_head + head_range_begin;
 
     // ---- per-lane column facts ---------------------------------------------------------------------------
-    auto column_token = [&](int nt) { return token_of_column(p, (wave * NTW + nt) * 16 + r16); };
-    auto column_head = [&](int nt) { return (wave * NTW + nt) * 16 + r16 - column_token(nt) * p.max_q_heads; };
+    // Twelve waves have 168 registers each: a column's token and head are worked out again where they are needed (a multiplication) instead
+    // of living through the tile loop.  Prompts of 24..500 tokens at Hq24/Hkv4/D256 on FP8 pages 0.9 % behind a division per column with
+    // them in registers, 1.4 % ahead without; decode beside two chunks on bf16 pages 106.9 -> 104.0 us.  The FP8 verify tiles lose 1 %.
+    auto column_of = [&](int nt) -> uint32_t {
+        uint32_t c = (wave * NTW + nt) * 16 + r16;
+        if constexpr (NWAVES == 12) asm volatile("" : "+v"(c));
+        return c;
+    };
+    auto column_token = [&](int nt) { return token_of_column(p, column_of(nt)); };
+    auto column_head = [&](int nt) { const uint32_t c = column_of(nt); return c - token_of_column(p, c) * p.max_q_heads; };
     uint32_t col_lo[NTW], col_hi[NTW];
     bool col_active[NTW];
     uint32_t blk_lo = 0xffffffffu, blk_hi = 0u, wave_all_lo = 0u, wave_all_hi = 0xffffffffu, min_span = 0xffffffffu;
