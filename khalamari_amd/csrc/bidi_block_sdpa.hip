@@ -17,6 +17,8 @@
 // maximum first, then weights, their sum and the weighted sum in key order.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "common.h"
 #include "device_math.hip.h"
 #include "device_params.h"
@@ -214,6 +216,17 @@ __global__ __launch_bounds__(kBidiThreads) void bidi_block_sdpa_kernel(const Bid
     }
 }
 
+// the larger of two bf16 magnitudes, in two positions
+__device__ __forceinline__ uint32_t max_u16x2(uint32_t a, uint32_t b) {
+    typedef unsigned short U16x2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(U16x2, a), __builtin_bit_cast(U16x2, b)));
+}
+// two bf16 values, zeros in the place of infinities and NaN
+__device__ __forceinline__ uint32_t without_infinities(uint32_t pair) {
+    const uint32_t low = (pair & 0x7f80u) == 0x7f80u ? 0u : pair & 0xffffu;
+    return low | ((pair & 0x7f800000u) == 0x7f800000u ? 0u : pair & 0xffff0000u);
+}
+
 // The same for bf16 rows of 128 or 256 dims and request blocks of at most sixteen tokens (what the executor drafts), on the matrix
 // cores: one wave per (Q range, KV head), four KV heads to a block, the wave's (token, Q head) tasks the columns of 16-wide tiles:
 //     S^T[16 keys][cols] = K . Q^T         v_mfma_f32_16x16x32_bf16, K and Q rows straight from memory
@@ -271,65 +284,82 @@ __global__ __launch_bounds__(kBidiHeadsPerBlock * 64) void bidi_block_sdpa_mfma_
 #pragma unroll
         for (int i = 0; i < 16 / ROWS_PER_LOAD; ++i)
             v_rows[i] = *reinterpret_cast<const uint4*>(local_v + row_of(i * ROWS_PER_LOAD + lane / CHUNKS) + (lane % CHUNKS) * 8);
+        uint32_t largest = 0;   // magnitude of the lane's V values, two positions
 #pragma unroll
-        for (int i = 0; i < 16 / ROWS_PER_LOAD; ++i)
+        for (int i = 0; i < 16 / ROWS_PER_LOAD; ++i) {
             *reinterpret_cast<uint4*>(v_tile + (i * ROWS_PER_LOAD + lane / CHUNKS) * V_ROW + (lane % CHUNKS) * 16) = v_rows[i];
+            largest = max_u16x2(max_u16x2(max_u16x2(max_u16x2(largest, v_rows[i].x & 0x7fff7fffu), v_rows[i].y & 0x7fff7fffu), v_rows[i].z & 0x7fff7fffu), v_rows[i].w & 0x7fff7fffu);
+        }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        for (uint32_t tile = 0; tile < num_tasks; tile += 16) {
-            const uint32_t task = tile + r16;
-            const bool live = task < num_tasks;
-            const uint32_t token_offset = live ? task / group : 0u;
-            const uint32_t q_token = token_lo + token_offset;
-            const uint32_t q_head = kv_head * group + (live ? task - token_offset * group : 0u);
-            const uint16_t* q_row = q + ((uint64_t)q_token * p.num_q_heads + q_head) * D + g * 8;
-            f32x4 s = {0.0f, 0.0f, 0.0f, 0.0f};
+        auto attend = [&](auto v_finite) __attribute__((always_inline)) {
+            for (uint32_t tile = 0; tile < num_tasks; tile += 16) {
+                const uint32_t task = tile + r16;
+                const bool live = task < num_tasks;
+                const uint32_t token_offset = live ? task / group : 0u;
+                const uint32_t q_token = token_lo + token_offset;
+                const uint32_t q_head = kv_head * group + (live ? task - token_offset * group : 0u);
+                const uint16_t* q_row = q + ((uint64_t)q_token * p.num_q_heads + q_head) * D + g * 8;
+                f32x4 s = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-            for (int ks = 0; ks < KS; ++ks)
-                s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, k_frag[ks]),
-                                                            __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(q_row + ks * 32)), s, 0, 0, 0);
-            // the four lanes of a column hold four keys each
-            float top = -INFINITY;
+                for (int ks = 0; ks < KS; ++ks)
+                    s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, k_frag[ks]),
+                                                                __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(q_row + ks * 32)), s, 0, 0, 0);
+                // the four lanes of a column hold four keys each
+                float top = -INFINITY;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                if ((uint32_t)(g * 4 + i) >= B) s[i] = -INFINITY;
-                top = fmaxf(top, s[i]);
+                for (int i = 0; i < 4; ++i) {
+                    if ((uint32_t)(g * 4 + i) >= B) s[i] = -INFINITY;
+                    top = fmaxf(top, s[i]);
+                }
+                top = max_over_rows(top);
+                float weight[4], sum = 0.0f;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    weight[i] = fast_exp2((s[i] - top) * scale_log2e);
+                    sum += weight[i];
+                }
+                sum = sum_over_rows(sum);
+                uint2 piece[3];
+#pragma unroll
+                for (int n = 0; n < 3; ++n) {
+                    piece[n] = make_uint2(pack_bf16x2(weight[0], weight[1]), pack_bf16x2(weight[2], weight[3]));
+                    weight[0] -= bf16_bits_to_f32(piece[n].x & 0xffffu);
+                    weight[1] -= bf16_bits_to_f32(piece[n].x >> 16);
+                    weight[2] -= bf16_bits_to_f32(piece[n].y & 0xffffu);
+                    weight[3] -= bf16_bits_to_f32(piece[n].y >> 16);
+                }
+                const uint64_t state = ((uint64_t)slot * p.num_q_heads + q_head) * p.max_q_tokens + (q_token - flat_begin);
+                const float inverse = sum > 0.0f ? 1.0f / sum : 0.0f;
+                if (live && g == 0) {
+                    p.exp_sums[state] = sum;
+                    p.max_logits[state] = top * p.scale;
+                }
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt) {
+                    uint2 a = __builtin_bit_cast(uint2, lds_read_tr16(v_transposed + mt * 32));   // keys 4 g .. 4 g + 3
+                    uint2 rest = a;
+                    if constexpr (!decltype(v_finite)::value) {
+                        const uint32_t keys = B - min((uint32_t)g * 4, B);
+                        a.x = keys >= 2 ? a.x : keys == 1 ? a.x & 0xffffu : 0u;
+                        a.y = keys >= 4 ? a.y : keys == 3 ? a.y & 0xffffu : 0u;
+                        rest = make_uint2(without_infinities(a.x), without_infinities(a.y));
+                    }
+                    f32x4 out = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                    for (int n = 2; n >= 0; --n)
+                        out = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, n > 0 ? rest : a), __builtin_bit_cast(s16x4, piece[n]), out, 0, 0, 0);
+                    if (live)
+                        *reinterpret_cast<uint2*>(partial + state * D + mt * 16 + g * 4) =
+                            make_uint2(pack_bf16x2(out[0] * inverse, out[1] * inverse), pack_bf16x2(out[2] * inverse, out[3] * inverse));
+                }
             }
-            top = max_over_rows(top);
-            float weight[4], sum = 0.0f;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                weight[i] = fast_exp2((s[i] - top) * scale_log2e);
-                sum += weight[i];
-            }
-            sum = sum_over_rows(sum);
-            uint2 piece[3];
-#pragma unroll
-            for (int n = 0; n < 3; ++n) {
-                piece[n] = make_uint2(pack_bf16x2(weight[0], weight[1]), pack_bf16x2(weight[2], weight[3]));
-                weight[0] -= bf16_bits_to_f32(piece[n].x & 0xffffu);
-                weight[1] -= bf16_bits_to_f32(piece[n].x >> 16);
-                weight[2] -= bf16_bits_to_f32(piece[n].y & 0xffffu);
-                weight[3] -= bf16_bits_to_f32(piece[n].y >> 16);
-            }
-            const uint64_t state = ((uint64_t)slot * p.num_q_heads + q_head) * p.max_q_tokens + (q_token - flat_begin);
-            const float inverse = sum > 0.0f ? 1.0f / sum : 0.0f;
-            if (live && g == 0) {
-                p.exp_sums[state] = sum;
-                p.max_logits[state] = top * p.scale;
-            }
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt) {
-                const s16x4 a = __builtin_bit_cast(s16x4, lds_read_tr16(v_transposed + mt * 32));
-                f32x4 out = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-                for (int n = 2; n >= 0; --n) out = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, __builtin_bit_cast(s16x4, piece[n]), out, 0, 0, 0);
-                if (live)
-                    *reinterpret_cast<uint2*>(partial + state * D + mt * 16 + g * 4) =
-                        make_uint2(pack_bf16x2(out[0] * inverse, out[1] * inverse), pack_bf16x2(out[2] * inverse, out[3] * inverse));
-            }
-        }
+        };
+        // An infinite value may meet the first piece of its own key's weight only: remainders may be zero or negative, and the weight
+        // of a key behind the block is zero.
+        if (__builtin_amdgcn_ballot_w64((largest & 0xffffu) >= 0x7f80u || (largest >> 16) >= 0x7f80u) == 0) attend(std::true_type{});
+        else attend(std::false_type{});
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();   // the next request block's V may replace this one's
     }

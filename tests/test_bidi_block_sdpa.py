@@ -173,6 +173,46 @@ def test_gpu_small_blocks_on_the_matrix_cores(device, hq, hkv, d, block, max_q):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("hq,hkv,d,block", [(8, 2, 128, 1), (40, 8, 128, 7), (24, 6, 128, 16), (48, 4, 256, 4), (16, 1, 256, 16), (6, 3, 96, 5)])
+def test_gpu_infinite_values_stay_infinite(device, hq, hkv, d, block):
+    """Every weight is positive, so an infinite value of any key makes its dimension infinite, two of opposite signs or a NaN make it NaN,
+    and the other dimensions, KV heads and request blocks keep their values.  The last key and a block of one key are in: weights of
+    exactly one and rows that the kernel for small blocks repeats (the last case runs the general kernel)."""
+    import torch
+
+    from khalamari_amd import bidi_block_sdpa as bb
+
+    requests = 3
+    tokens = requests * block
+    rng = np.random.default_rng(hq + block)
+    q, k, v = (oracle.bf16_round(rng.standard_normal((tokens, heads, d)).astype(np.float32)) for heads in (hq, hkv, hkv))
+    last = block - 1                       # of the first request block; the second has opposite infinities, the third none
+    v[last, 0, 0], v[last, 0, 77], v[0, hkv - 1, 5], v[last, 0, 40] = np.inf, -np.inf, -np.inf, np.nan
+    v[block, 0, 3], v[2 * block - 1, 0, 3], v[2 * block - 1, 0, d - 1] = -np.inf, np.inf, np.inf
+    ranges = np.array([[r * block, (r + 1) * block] for r in range(requests)], dtype=np.uint32)
+    cu = np.arange(requests + 1, dtype=np.uint32)
+    scale = float(np.float32(d) ** np.float32(-0.5))
+    config, shape = bb.Config(block, block, hq, hkv, d, scale, DTYPE_BF16), bb.Shape(tokens, requests, requests)
+    stats = config.partial_output_stat_elements(shape)
+    sums, maxs = (torch.zeros(stats, dtype=torch.float32, device=device) for _ in range(2))
+    partial = torch.zeros(config.partial_output_values(shape) * 2, dtype=torch.uint8, device=device)
+    print(f"bidi block infinities: hq={hq} hkv={hkv} d={d} block={block}", flush=True)
+    bits = oracle.f32_to_bf16_bits
+    bb.Compute(config).invoke(shape, ReplayU32.fixed(requests), q=_to(device, bits(q)), local_k=_to(device, bits(k)), local_v=_to(device, bits(v)),
+                              q_token_ranges=_to(device, ranges), cu_sdpa_partial_outputs=_to(device, cu), partial_exp_sums=sums,
+                              partial_max_logits=maxs, partial_output=partial)
+    torch.cuda.synchronize()
+    with np.errstate(invalid="ignore"):
+        want = oracle.bidi_block_sdpa(q, k, v, ranges, cu, requests, block, block, hq, hkv, d, scale, requests)[2]
+    got = oracle.bf16_bits_to_f32(partial.cpu().numpy().view(np.uint16)).reshape(want.shape)
+    assert np.isinf(want).any() and np.isnan(want).any()
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(np.isinf(got), np.isinf(want)) and np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
+    finite = np.isfinite(want)
+    assert np.abs(got[finite] - want[finite]).max() < 1e-2
+
+
+@pytest.mark.gpu
 def test_gpu_replay_active_q_token_ranges(device):
     """test_replay_active_q_token_ranges_match_cpu_reference (bidi_block_sdpa_test.rs:50-157)."""
     import torch
