@@ -679,7 +679,8 @@ int khm_selection_cu_partial_outputs(const khm_selection* selection, uint32_t* o
  * selection.  update() fills one of three blocks of pinned staging memory and enqueues one kernel on `stream` that
  * copies it to the device arrays (the reference writes shared-memory buffers directly); arrays the reference leaves
  * untouched stay untouched (q_token_ranges for the sliced-KV kind, every tail beyond the written prefix).  It does not
- * wait for `stream`, only for the copy of three updates ago; a stream that is being captured is refused.
+ * wait for `stream`, only for the copy of three updates ago (a stream of another device than create()'s takes copies and is
+ * waited for); a stream that is being captured is refused.
  * create() and destroy() allocate and free device and pinned memory, and update() may wait for a copy: none of the three
  * may run while any stream of the process is under hipGraph capture in the global mode (the capture is invalidated and
  * its next enqueue fails).  A host language with finalizers must not leave destroy() to its collector. */

@@ -138,6 +138,7 @@ struct khm_gqa_metadata {
     uint32_t* device[kNumArrays] = {};
     StagingBlock staging[kStagingBlocks];
     int next_block = 0;
+    int device_id = 0;                   // the device that was current in create()
 };
 
 extern "C" void khm_gqa_metadata_destroy(khm_gqa_metadata* metadata) {
@@ -169,7 +170,7 @@ extern "C" int khm_gqa_metadata_create(uint64_t max_tokens, uint64_t max_map_tas
     metadata->capacity[KHM_METADATA_SDPA_MAP_TASK_TEMPLATES] = max_map_task_templates * 3;
     metadata->capacity[KHM_METADATA_CU_SDPA_PARTIAL_OUTPUTS] = max_tokens + 1;
     uint64_t block_words = 0;
-    hipError_t status = hipSuccess;
+    hipError_t status = hipGetDevice(&metadata->device_id);
     for (int i = 0; i < kNumArrays && status == hipSuccess; ++i) {
         const size_t bytes = metadata->capacity[i] * sizeof(uint32_t);
         status = hipMalloc(reinterpret_cast<void**>(&metadata->device[i]), bytes);
@@ -224,6 +225,23 @@ extern "C" int khm_gqa_metadata_update(khm_gqa_metadata* metadata, const uint32_
         p.end[i] = total;
     }
     if (total == 0) return KHM_OK;
+    // The kernel writes memory of the object's device and the event is recorded there.  A stream of another device (the null stream, while
+    // another device is current) takes copies, which may cross devices, and is waited for.
+    int stream_device = -1;
+    status = stream != nullptr ? hipStreamGetDevice(static_cast<hipStream_t>(stream), &stream_device) : hipGetDevice(&stream_device);
+    if (status != hipSuccess || stream_device != metadata->device_id) {
+        (void)hipGetLastError();
+        status = hipSuccess;
+        for (int i = 0; i < kNumArrays && status == hipSuccess; ++i) {
+            const uint64_t begin = i > 0 ? p.end[i - 1] : 0;
+            if (p.end[i] > begin)
+                status = hipMemcpyAsync(p.target[i], p.source + begin, (p.end[i] - begin) * sizeof(uint32_t), hipMemcpyHostToDevice, static_cast<hipStream_t>(stream));
+        }
+        const hipError_t waited = hipStreamSynchronize(static_cast<hipStream_t>(stream));
+        if (status == hipSuccess) status = waited;
+        if (status != hipSuccess) return fail(KHM_ERR_HIP, "GQA batch metadata upload failed: %s", hipGetErrorString(status));
+        return KHM_OK;
+    }
     KHM_LAUNCH(upload_metadata_kernel, dim3((uint32_t)((total + 255) / 256)), dim3(256), 0, static_cast<hipStream_t>(stream), p);
     status = hipGetLastError();
     if (status == hipSuccess) status = hipEventRecord(block.copied, static_cast<hipStream_t>(stream));

@@ -64,3 +64,23 @@ def test_an_update_is_not_captured(device):
     assert len(refused) == 1 and "stream wait failed" in refused[0]
     metadata.update([0, 1, 2, 3], [5, 6, 7, 8], [0, 1, 2, 3, 4], selection)
     torch.cuda.synchronize()
+
+
+@pytest.mark.skipif(torch.cuda.device_count() < 2, reason="two GPUs")
+@pytest.mark.parametrize("own_stream", [False, True])
+def test_an_update_on_a_stream_of_another_device(device, own_stream):
+    """The arrays are the first device's; the update is called with the second one current."""
+    selector = _selector(4)
+    limits = selector.limits()
+    with torch.cuda.device(0):
+        metadata = batch_metadata.GQAMetadataBuffers(limits.max_tokens, limits.max_map_task_templates)
+        views = [torch.as_tensor(_View(metadata.buffer(i)), device="cuda:0") for i in range(6)]
+    policy = GQAReplayBucketPolicy(limits.max_tokens, limits.max_map_task_templates)
+    with torch.cuda.device(1):
+        for step in range(5):
+            histories = [step, step + 1, step + 2, step + 3]
+            selection = selector.select(RequestShape.from_batch(histories, [0, 1, 2, 3, 4]), policy, 4)
+            metadata.update([0, 1, 2, 3], histories, [0, 1, 2, 3, 4], selection, stream=torch.cuda.Stream() if own_stream else None)
+            torch.cuda.synchronize()
+            for i in range(6):
+                assert np.array_equal(views[i].cpu().numpy().view(np.uint32), metadata.host(i)), (step, i)
