@@ -6,6 +6,7 @@
 // staged in a ring of pinned host blocks, from which one small kernel on the caller's stream copies them to the device arrays.
 #include <hip/hip_runtime.h>
 
+#include <new>
 #include <vector>
 
 #include "common.h"
@@ -184,11 +185,15 @@ extern "C" int khm_gqa_metadata_create(uint64_t max_tokens, uint64_t max_map_tas
         if (status == hipSuccess) status = hipHostMalloc(reinterpret_cast<void**>(&block.words), block_words * sizeof(uint32_t), hipHostMallocCoherent);
         if (status == hipSuccess) status = hipEventCreateWithFlags(&block.copied, hipEventDisableTiming);
     }
+    try {
+        for (int i = 0; i < kNumArrays && status == hipSuccess; ++i) metadata->host[i].assign(metadata->capacity[i], 0u);
+    } catch (const std::bad_alloc&) {   // no exception leaves a C entry
+        status = hipErrorOutOfMemory;
+    }
     if (status != hipSuccess) {
         khm_gqa_metadata_destroy(metadata);
         return fail(KHM_ERR_HIP, "GQA batch metadata allocation failed: %s", hipGetErrorString(status));
     }
-    for (int i = 0; i < kNumArrays; ++i) metadata->host[i].assign(metadata->capacity[i], 0u);
     *out = metadata;
     return KHM_OK;
 }
