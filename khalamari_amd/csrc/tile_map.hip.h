@@ -786,9 +786,10 @@ void tile_map_kernel(const MapParams p) {
     };
     Scores pending;
     TileIds upcoming = fetch_ids(NSTAGES - 1);
-    // FP8 pages: decode tile + 2 from registers into LDS, request tile + 3.  The MFMA-bound tiles (two column tiles per
-    // wave) do it behind the first S^T of the tile like the bf16 path requests its loads (1.6 % on config 5); the
-    // bandwidth-bound verify tiles do it straight after the barrier, where the decoded tile is ready soonest (2 %).
+    // Register-staged FP8 tiles: decode tile + 2 from registers into LDS, request tile + 3.  Tiles with two column tiles per wave do it
+    // behind the first S^T of the tile like the bf16 path requests its loads (1.6 % on config 5); those with one (head dim 256) straight
+    // after the barrier: four chunks of 1000..2048 tokens on up to 8000 at Hq24/Hkv4 985 us, behind the scores 1062 (prompts of 20..900
+    // tokens there 226 us, behind the scores 187; at Hq16/Hkv2 no difference).
     constexpr bool kRawTileBehindScores = NTW >= 2;
     auto advance_raw_tiles = [&](uint32_t tile) __attribute__((always_inline)) {
         if (tile + 2 < num_tiles) write_raw_tile(tile + 2);
