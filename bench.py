@@ -32,7 +32,7 @@ NUM_POOLS = 3
 # two `rocprofv3 --pmc` runs per config, each counter scaled by what it reads for a plain 1 GiB copy kernel
 # (`--calibration-copy`).  The summaries with their commands are the text files under profiles/.
 MEASURED_MAP_TRAFFIC_BYTES = {2: 565_561_344, 3: 2_153_930_752, 4: 1_446_890_496, 5: 1_202_827_264, 6: 1_068_915_712}
-MEASURED_MAP_TRAFFIC_BYTES_FP8_PAGES = {2: 286_631_936, 3: 1_082_411_008, 4: 729_135_104, 5: 869_629_952, 6: 1_614_041_088}
+MEASURED_MAP_TRAFFIC_BYTES_FP8_PAGES = {2: 286_631_936, 3: 1_082_411_008, 4: 729_135_104, 5: 869_629_952, 6: 1_592_212_216}
 
 CONFIGS = {
     1: dict(name="config1: B=1 q=1 Hq32/Hkv8/D128 ctx 1024, identity pages", hq=32, hkv=8, d=128, kind="decode", kv_slice=64),
